@@ -216,8 +216,9 @@ class LaunchGeometry:
     rows_symbol: str = "M"
     nnz_chunk: int = 0
     stream: bool = False
+    helper_div: int = 0
 
-    def grid(self, rows: int, nnz: int = 0) -> int:
+    def grid(self, rows: int, nnz: int = 0, K: int = 64) -> int:
         if rows <= 0:
             return 0
         if self.stream:
@@ -225,6 +226,11 @@ class LaunchGeometry:
         g = (int(rows) + self.rows_per_block - 1) // self.rows_per_block
         if self.nnz_chunk:
             g += max(0, int(nnz)) // self.nnz_chunk + 1
+        if self.helper_div and K > SPMM_WAVE_K:
+            hr = spmm_helper_rows(int(rows), self.helper_div)
+            help_ = SPMM_SLICES * ((int(rows) + hr - 1) // hr)
+            if (g + help_) * self.block <= 0xFFFFFFFF:
+                g += help_
         return g
 
     def to_dict(self) -> Dict[str, Any]:
@@ -234,6 +240,8 @@ class LaunchGeometry:
             d["nnz_chunk"] = self.nnz_chunk
         if self.stream:
             d["stream"] = True
+        if self.helper_div:
+            d["helper_div"] = self.helper_div
         return d
 
 
@@ -754,9 +762,15 @@ def launch_geometry(plan: Plan, low: Lowering) -> LaunchGeometry:
         lists = [(4, rows), (4, 1), (8, 1)] if low.tiled else []
         return LaunchGeometry(rows, B, _lds_total(lists + lists), plan.row_extent)
     if plan.kind == "row_dense_out":
+        if not low.tiled:
+            return LaunchGeometry(rows, B, 0, plan.row_extent)
         V = 2 if low.vector_width >= 2 else 1
-        arrays = [(4, rows), (4, 1), (8, B * V), (8, 1)] if low.tiled else []
-        return LaunchGeometry(rows, B, _lds_total(arrays), plan.row_extent)
+        # row pointers, a row's first and last column, the tile's nonzeros, listed and
+        # dwarfing rows and their counts, the skew flag, the helpers' row bits, partial C-row slices
+        arrays = [(8, rows + 1), (8, 2), (8, 1), (4, rows), (4, 1), (4, rows // 4 + 1), (4, 1),
+                  (4, 1), (8, SPMM_HELP_MAX // 64), (8, spmm_part(B, V))]
+        return LaunchGeometry(rows, B, _lds_total(arrays), plan.row_extent,
+                            helper_div=spmm_helper_div(B))
     if plan.kind != "scalar_reduce" or not low.tiled:
         return LaunchGeometry(rows, B, 0, plan.row_extent)
     if low.balance == "stream":
@@ -787,6 +801,46 @@ def module_scratch(plan: Plan, low: Lowering) -> bool:
     must not overlap on one device."""
     return (plan.kind == "scalar_reduce" and low.tiled
             and low.balance in ("nnz", "hybrid", "stream"))
+
+
+# Tiled SpMM's paths over staged row pointers (_SPMM_WAVE) run at K over SPMM_WAVE_K.  A row of more than
+# spmm_huge nonzeros that is also over four times its tile's average is summed by
+# SPMM_SLICES helper workgroups, a quarter of the columns each.
+SPMM_WAVE_K = 16
+SPMM_SLICES = 4
+
+
+def spmm_helper_div(block: int) -> int:
+    """Rows are dealt to about this many groups of helpers: one per CU where a helper has
+    8 waves or more, half of that where its few waves leave each scan longer and more
+    helpers would crowd out tiles that are all resident at once."""
+    return 256 if block >= 512 else 128
+
+
+SPMM_HELP_MAX = 1024
+
+
+def spmm_helper_rows(rows: int, div: int) -> int:
+    """Rows whose pointers one helper scans, whole 64-lane ballots of them."""
+    return min(SPMM_HELP_MAX, max(64, (rows // div + 63) // 64 * 64))
+
+
+def spmm_huge(block: int, unroll: int) -> int:
+    """Nonzeros past which a row may go to the helpers: two per lane of the
+    workgroup, and never fewer than a row listed as long has."""
+    return max(2 * block, 16 * unroll)
+
+
+def spmm_cols(V: int) -> int:
+    """Columns per pass of the wave path's widest form: 64 lanes, four each."""
+    return 256
+
+
+def spmm_part(block: int, V: int) -> int:
+    """Doubles of the partial C-row slices: one slice per lane group, or two rows'
+    pieces per wave on the wave path."""
+    waves = block // WAVE
+    return max(block * V, 2 * waves * spmm_cols(V) if waves > 1 else 0)
 
 
 # Stream ranges: at most this many nonzeros per workgroup (their products are
@@ -2410,8 +2464,499 @@ def _value_with(plan: Plan, data_text: str, gathered_text: str, row: str, col_te
     return rec(plan.value_expr)
 
 
+_SPMM_WAVE = r"""
+// Value of v held by lane src (uniform) of the wave.
+__device__ __forceinline__ tg_i64 tg_lane_read(tg_i64 v, int src) {
+  const int lo = __builtin_amdgcn_readlane((int)v, src);
+  const int hi = __builtin_amdgcn_readlane((int)(v >> 32), src);
+  return ((tg_i64)hi << 32) | (tg_i64)(unsigned)lo;
+}
+__device__ __forceinline__ double tg_lane_read(double v, int src) {
+  return __longlong_as_double(tg_lane_read((tg_i64)__double_as_longlong(v), src));
+}
+
+// CL neighbouring columns of a lane; a pair needs 8-byte alignment only (gfx950 loads
+// and stores 128 bits at any 4-byte boundary), so odd K and sub-buffers take pairs too.
+template <int CL> struct tg_cols;
+template <> struct tg_cols<1> {
+  typedef double t;
+  static __device__ __forceinline__ double get(double v, int) { return v; }
+};
+template <> struct tg_cols<2> {
+  typedef double t __attribute__((ext_vector_type(2), aligned(8)));
+  static __device__ __forceinline__ double get(t v, int c) { return c ? v.y : v.x; }
+};
+
+// Wave path of SpMM: the tile's nonzeros (but those of the rows listed in s_huge) are cut
+// into one equal run per wave, and a wave walks its run in position order with all 64 lanes
+// on one nonzero's B row: 64 CL E columns a pass, U nonzeros' loads in flight.  Column and
+// value of 64 positions are loaded at once, one per lane, and read back with v_readlane, so
+// a B row's address is scalar.  A row inside the run is stored straight from the registers;
+// the pieces of a row cut at a run's ends go to s_part (slot 0: the piece of the row that
+// began before the run, slot 1: of the row that runs past its end) and the wave the row ends
+// in adds them in wave order after one barrier.
+// Bound by gathers: 1.6 M nonzeros over 130 columns take 271 us, 1.95 GB in lines from the
+// Infinity Cache; 4 to 16 nonzeros in flight per wave keep the kernel at 72 VGPRs, 7 waves
+// per SIMD, which the lane groups' paths need more than this one does (98 us at 7, 122 at 6).
+template <int CL, int E, int U, int WAVES>
+__device__ __forceinline__ void tg_spmm_wave(
+    const tg_i64* __restrict__ indices, const double* __restrict__ data,
+    const double* __restrict__ Bm, double* __restrict__ C, const tg_i64 K, const tg_i64 row0,
+    const int nrows, const tg_i64* s_ptr, const int* s_huge, const int nh, double* s_part,
+    const int wv) {
+  typedef typename tg_cols<CL>::t cols;
+  constexpr int NC = 64 * CL * E;
+  const int l = threadIdx.x & 63;
+  const tg_i64 glo = tg_uniform(s_ptr[0]);
+  tg_i64 L = tg_uniform(s_ptr[nrows]) - glo;   // positions shared out
+  #pragma unroll 1
+  for (int h = 0; h < nh; ++h) {
+    const int i = __builtin_amdgcn_readfirstlane(s_huge[h]);
+    L -= tg_uniform(s_ptr[i + 1]) - tg_uniform(s_ptr[i]);
+  }
+  const tg_i64 a = L * wv / WAVES, b = L * (wv + 1) / WAVES;
+  // rows without nonzeros
+  #pragma unroll 1
+  for (int i0 = wv * 64; i0 < nrows; i0 += 64 * WAVES) {
+    const int i = i0 + l;
+    unsigned long long m = __ballot(i < nrows && s_ptr[i < nrows ? i + 1 : 0] == s_ptr[i < nrows ? i : 0]);
+    #pragma unroll 1
+    for (; m; m &= m - 1) {
+      double* c = C + (row0 + i0 + (int)__builtin_ctzll(m)) * K;
+      for (tg_i64 k = l; k < K; k += 64) __builtin_nontemporal_store(0.0, c + k);
+    }
+  }
+  // position a of the run, huge rows skipped
+  tg_i64 x0 = glo + a;
+  #pragma unroll 1
+  for (int h = 0; h < nh; ++h) {
+    const int i = __builtin_amdgcn_readfirstlane(s_huge[h]);
+    const tg_i64 hs = tg_uniform(s_ptr[i]);
+    tg_i64 hc = hs - glo;   // its start among the shared positions
+    for (int g = 0; g < nh; ++g) {
+      const int j = __builtin_amdgcn_readfirstlane(s_huge[g]);
+      if (j < i) hc -= tg_uniform(s_ptr[j + 1]) - tg_uniform(s_ptr[j]);
+    }
+    if (hc <= a) x0 += tg_uniform(s_ptr[i + 1]) - hs;
+  }
+  #pragma unroll 1
+  for (tg_i64 kb = 0; kb < K; kb += NC) {
+    // column offsets from kbase; a lane past the last columns loads the last ones again
+    const tg_i64 kbase = kb >= 2 ? kb - 2 : 0;
+    unsigned ko[E];
+    bool st1[E], stc[E];   // the lane has a column, has all CL of them
+    #pragma unroll
+    for (int e = 0; e < E; ++e) {
+      tg_i64 k = kb + e * 64 * CL + l * CL;
+      st1[e] = k < K;
+      stc[e] = k + CL <= K;
+      if (!stc[e]) k = K - CL;
+      ko[e] = (unsigned)(k - kbase) * 8u;
+    }
+    const char* const Bk = (const char*)(Bm + kbase);
+    double acc[E][CL];
+    #pragma unroll
+    for (int e = 0; e < E; ++e)
+      #pragma unroll
+      for (int c = 0; c < CL; ++c) acc[e][c] = 0.0;
+    int r = 0;            // row of the walk, and the first one
+    int rf = 0;
+    bool cut = false;     // row rf began before this run
+    bool fin = false;     // and ended in it
+    tg_i64 cur = x0, rem = b - a;
+    auto store = [&](int row) {
+      char* const c = (char*)(C + (row0 + row) * K + kbase);
+      #pragma unroll
+      for (int e = 0; e < E; ++e) {
+        if (CL == 2) {
+          if (stc[e]) {
+            typename tg_cols<2>::t v;
+            v.x = acc[e][0];
+            v.y = acc[e][CL - 1];
+            __builtin_nontemporal_store(v, (typename tg_cols<2>::t*)(c + ko[e]));
+          } else if (st1[e]) {
+            __builtin_nontemporal_store(acc[e][CL - 1], (double*)(c + ko[e]) + 1);
+          }
+        } else if (st1[e]) {
+          __builtin_nontemporal_store(acc[e][0], (double*)(c + ko[e]));
+        }
+      }
+    };
+    auto part = [&](int slot) {
+      double* const p = s_part + (wv * 2 + slot) * NC + l * CL;
+      #pragma unroll
+      for (int e = 0; e < E; ++e)
+        #pragma unroll
+        for (int c = 0; c < CL; ++c) p[e * 64 * CL + c] = acc[e][c];
+    };
+    #pragma unroll 1
+    while (rem > 0) {
+      tg_i64 y = cur + rem;
+      #pragma unroll 1
+      for (int h = 0; h < nh; ++h) {
+        const tg_i64 hs = tg_uniform(s_ptr[__builtin_amdgcn_readfirstlane(s_huge[h])]);
+        if (hs >= cur && hs < y) y = hs;
+      }
+      if (y > cur) {
+        // the row holding cur, and the ends of the rows from it on, one per lane
+        r = 0;
+        #pragma unroll 1
+        for (int i0 = 0; i0 < nrows; i0 += 64) {
+          const int i = i0 + l;
+          const unsigned long long m = __ballot(i < nrows && s_ptr[i < nrows ? i + 1 : 0] <= cur);
+          r += (int)__builtin_popcountll(m);
+          if (~m) break;
+        }
+        int rb = r;
+        tg_i64 ends = s_ptr[rb + 1 + l < nrows ? rb + 1 + l : nrows];
+        if (cur == x0) {
+          rf = r;
+          cut = tg_uniform(s_ptr[r]) < cur;
+        }
+        tg_i64 rend64 = tg_lane_read(ends, 0);
+        tg_i64 jl = indices[cur + l < y ? cur + l : cur] * K * 8;
+        double vl = data[cur + l < y ? cur + l : cur];
+        #pragma unroll 1
+        for (tg_i64 pc = cur; pc < y; pc += 64) {
+          const int n = (int)(y - pc < 64 ? y - pc : 64);
+          int rend = (int)(rend64 - pc < 127 ? rend64 - pc : 127);
+          tg_i64 jn = 0;
+          double vn = 0.0;
+          if (pc + 64 < y) {
+            const tg_i64 q = pc + 64 + l < y ? pc + 64 + l : cur;
+            jn = indices[q] * K * 8;
+            vn = data[q];
+          }
+          #pragma unroll 1
+          for (int s = 0; s < n; s += U) {
+            cols v[U][E];
+            #pragma unroll
+            for (int u = 0; u < U; ++u) {
+              const char* const br = Bk + tg_lane_read(jl, s + u < n ? s + u : n - 1);
+              #pragma unroll
+              for (int e = 0; e < E; ++e) v[u][e] = *(const cols*)(br + ko[e]);
+            }
+            #pragma unroll
+            for (int u = 0; u < U; ++u) {
+              if (s + u < n) {
+                const double d = tg_lane_read(vl, s + u);
+                #pragma unroll
+                for (int e = 0; e < E; ++e)
+                  #pragma unroll
+                  for (int c = 0; c < CL; ++c) acc[e][c] += d * tg_cols<CL>::get(v[u][e], c);
+                if (s + u + 1 == rend) {   // the row's last nonzero
+                  if (WAVES > 1 && cut && r == rf) {
+                    part(0);
+                    fin = true;
+                  } else {
+                    store(r);
+                  }
+                  #pragma unroll
+                  for (int e = 0; e < E; ++e)
+                    #pragma unroll
+                    for (int c = 0; c < CL; ++c) acc[e][c] = 0.0;
+                  const tg_i64 here = rend64;
+                  #pragma unroll 1
+                  do {   // the next row with nonzeros
+                    ++r;
+                    if (r - rb >= 64) {
+                      rb = r;
+                      ends = s_ptr[rb + 1 + l < nrows ? rb + 1 + l : nrows];
+                    }
+                    rend64 = tg_lane_read(ends, r - rb);
+                  } while (r < nrows && rend64 == here);
+                  rend = (int)(rend64 - pc < 127 ? rend64 - pc : 127);
+                }
+              }
+            }
+          }
+          jl = jn;
+          vl = vn;
+        }
+        if (WAVES > 1 && r < nrows && y - cur == rem && tg_uniform(s_ptr[r]) < y)
+          part(cut && r == rf ? 0 : 1);   // the run ends inside row r
+      }
+      rem -= y - cur;
+      cur = y;
+      #pragma unroll 1
+      for (int h = 0; h < nh; ++h) {
+        const int i = __builtin_amdgcn_readfirstlane(s_huge[h]);
+        if (tg_uniform(s_ptr[i]) == y) cur = tg_uniform(s_ptr[i + 1]);
+      }
+    }
+    if (WAVES > 1) {
+      __syncthreads();
+      if (fin) {
+        // row rf began in wave s's run (the last whose run starts at or before the row)
+        tg_i64 c0 = tg_uniform(s_ptr[rf]) - glo;
+        #pragma unroll 1
+        for (int h = 0; h < nh; ++h) {
+          const int i = __builtin_amdgcn_readfirstlane(s_huge[h]);
+          if (i < rf) c0 -= tg_uniform(s_ptr[i + 1]) - tg_uniform(s_ptr[i]);
+        }
+        int s = wv - 1;
+        while (s > 0 && L * s / WAVES > c0) --s;
+        #pragma unroll 1
+        for (int i = s; i <= wv; ++i) {
+          if (L * i / WAVES == L * (i + 1) / WAVES) continue;   // an empty run
+          const double* const p = s_part + (i * 2 + (i == s ? 1 : 0)) * NC + l * CL;
+          #pragma unroll
+          for (int e = 0; e < E; ++e)
+            #pragma unroll
+            for (int c = 0; c < CL; ++c) {
+              const double t = p[e * 64 * CL + c];
+              acc[e][c] = i == s ? t : acc[e][c] + t;
+            }
+        }
+        store(rf);
+      }
+      if (kb + NC < K) __syncthreads();
+    }
+  }
+}
+
+// Lane groups of SpMM: TPR lanes per row, CL E columns each from column kb on, the tile's
+// rows SLOTS apart, U nonzeros' B rows in flight.
+template <int TPR, int CL, int E, int U, int SLOTS>
+__device__ __forceinline__ void tg_spmm_rows(
+    const tg_i64* __restrict__ indices, const double* __restrict__ data,
+    const double* __restrict__ Bm, double* __restrict__ C, const tg_i64 K, const tg_i64 row0,
+    const int nrows, const tg_i64* s_ptr, const tg_i64 kb) {
+  typedef typename tg_cols<CL>::t cols;
+  const int lane = threadIdx.x % TPR;
+  // columns from kbase; a lane past the last columns loads the last ones again
+  const tg_i64 kbase = kb >= 2 ? kb - 2 : 0;
+  unsigned ko[E];
+  bool st1[E], stc[E];
+  #pragma unroll
+  for (int e = 0; e < E; ++e) {
+    const tg_i64 k = kb + e * TPR * CL + lane * CL;
+    st1[e] = k < K;
+    stc[e] = k + CL <= K;
+    ko[e] = (unsigned)((stc[e] ? k : K - CL) - kbase);
+  }
+  #pragma unroll 1
+  for (int r = threadIdx.x / TPR; r < nrows; r += SLOTS) {
+    const tg_i64 rs = s_ptr[r], re = s_ptr[r + 1];
+    double acc[E][CL];
+    #pragma unroll
+    for (int e = 0; e < E; ++e)
+      #pragma unroll
+      for (int c = 0; c < CL; ++c) acc[e][c] = 0.0;
+    #pragma unroll 1
+    for (tg_i64 p = rs; p < re; p += U) {
+      tg_i64 j[U];
+      double d[U];
+      cols v[U][E];
+      #pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const tg_i64 q = p + u < re ? p + u : p;
+        j[u] = indices[q];
+        d[u] = data[q];
+      }
+      #pragma unroll
+      for (int u = 0; u < U; ++u)
+        #pragma unroll
+        for (int e = 0; e < E; ++e) v[u][e] = *(const cols*)(Bm + kbase + j[u] * K + ko[e]);
+      #pragma unroll
+      for (int u = 0; u < U; ++u)
+        #pragma unroll
+        for (int e = 0; e < E; ++e)
+          #pragma unroll
+          for (int c = 0; c < CL; ++c)
+            acc[e][c] = p + u < re ? acc[e][c] + d[u] * tg_cols<CL>::get(v[u][e], c) : acc[e][c];
+    }
+    double* const c = C + (row0 + r) * K + kbase;
+    #pragma unroll
+    for (int e = 0; e < E; ++e) {
+      if (CL == 2 && stc[e]) {
+        typename tg_cols<2>::t t;
+        t.x = acc[e][0];
+        t.y = acc[e][CL - 1];
+        __builtin_nontemporal_store(t, (typename tg_cols<2>::t*)(c + ko[e]));
+      } else if (st1[e]) {
+        __builtin_nontemporal_store(acc[e][CL - 1], c + ko[e] + CL - 1);
+      }
+    }
+  }
+}
+"""
+
+
+def _spmm_helpers(w: _W, plan: Plan, low: Lowering, geo: LaunchGeometry, out_name: str,
+                  b_name: str, kext: str) -> None:
+    """The helper workgroups of a tiled SpMM kernel, ahead of its tiles, and the tiles' row0."""
+    B, TR, U = geo.block, geo.rows_per_block, max(1, low.unroll)
+    WAVES, NS = B // WAVE, SPMM_SLICES
+    LH = spmm_huge(B, U)
+    w("const unsigned tn = (unsigned)((%s + %d) / %d);  // tiles" % (plan.row_extent, TR - 1, TR))
+    w("int hr = %s < %dLL ? (int)(%s / %d + 63) / 64 * 64 : %d;  // rows per helper"
+      % (plan.row_extent, SPMM_HELP_MAX * geo.helper_div, plan.row_extent, geo.helper_div,
+         SPMM_HELP_MAX))
+    w("hr = hr < 64 ? 64 : hr;")
+    w("unsigned n_help = (unsigned)((%s + hr - 1) / hr) * %d;" % (plan.row_extent, NS))
+    w("if (((tg_i64)tn + n_help) * %d > 0xFFFFFFFFLL) n_help = 0;  // past one launch's work-items" % B)
+    w("__shared__ unsigned long long s_hrow[%d];  // a helper's rows, one bit each" % (SPMM_HELP_MAX // 64))
+    w.open("if (blockIdx.x < n_help)")
+    w("// Helper: of its hr rows, those over %d nonzeros and over 4 times their tile's" % LH)
+    w("// average.  %d helpers share hr rows: each a slice of the columns, or, with fewer" % NS)
+    w("// slices of 16 than helpers, every other of those rows.  16 columns at a time, each")
+    w("// group of 16 lanes on its own nonzeros and the groups' sums added in order")
+    w("const tg_i64 hr0 = (tg_i64)(blockIdx.x / %d) * hr;" % NS)
+    w("const tg_i64 sw = (%s + %d) / %d * 16;" % (kext, 16 * NS - 1, 16 * NS))
+    w("const int ns = %s <= 16 * %d ? (int)((%s + 15) / 16) : %d;" % (kext, NS, kext, NS))
+    w("const int sl = (int)(blockIdx.x %% %d), parts = %d / ns;" % (NS, NS))
+    w("const tg_i64 klo = (sl % ns) * sw;")
+    w("const tg_i64 khi = klo + sw < %s ? klo + sw : %s;" % (kext, kext))
+    w("if (klo >= khi || sl >= ns * parts || row_end <= 0) return;")
+    w("#pragma unroll 4")
+    w.open("for (int t = threadIdx.x; t < hr; t += %d)" % B)
+    w("const tg_i64 r = hr0 + t < row_end ? hr0 + t : row_end - 1;")
+    w("const tg_i64 n = indptr[r + 1] - indptr[r];")
+    w("bool big = n > %d && hr0 + t < row_end;" % LH)
+    w.open("if (big)")
+    w("const tg_i64 t0 = r / %d * %d, t1 = t0 + %d < row_end ? t0 + %d : row_end;" % (TR, TR, TR, TR))
+    w("big = n * (t1 - t0) > 4 * (indptr[t1] - indptr[t0]);")
+    w.close()
+    w("const unsigned long long m = __ballot(big);")
+    w("if ((threadIdx.x & 63) == 0) s_hrow[t >> 6] = m;")
+    w.close()
+    w("__syncthreads();")
+    w("const int q = threadIdx.x & 15, grp = threadIdx.x >> 4;")
+    w("int nth = 0;")
+    w("#pragma unroll 1")
+    w.open("for (int i0 = 0; i0 < hr / 64; ++i0)")
+    w("unsigned long long m = (unsigned long long)tg_uniform((tg_i64)s_hrow[i0]);")
+    w("#pragma unroll 1")
+    w.open("for (; m; m &= m - 1)")
+    w("if (nth++ % parts != sl / ns) continue;")
+    w("const tg_i64 row = hr0 + i0 * 64 + (int)__builtin_ctzll(m);")
+    w("const tg_i64 rs = tg_uniform(indptr[row]), re = tg_uniform(indptr[row + 1]);")
+    w("#pragma unroll 1")
+    w.open("for (tg_i64 kc = klo; kc < khi; kc += 16)")
+    w("const tg_i64 k = kc + q < khi ? kc + q : khi - 1;")
+    w("double acc = 0.0;")
+    w("#pragma unroll 1")
+    w.open("for (tg_i64 p = rs + grp; p < re; p += %d)" % (8 * (B // 16)))
+    w("tg_i64 j[8]; double v[8], b[8];")
+    w("#pragma unroll")
+    w.open("for (int u = 0; u < 8; ++u)")
+    w("const tg_i64 pu = p + u * %d < re ? p + u * %d : p;" % (B // 16, B // 16))
+    w("j[u] = indices[pu]; v[u] = data[pu];")
+    w.close()
+    w("#pragma unroll")
+    w("for (int u = 0; u < 8; ++u) b[u] = %s[j[u] * %s + k];" % (b_name, kext))
+    w("#pragma unroll")
+    w("for (int u = 0; u < 8; ++u) acc = p + u * %d < re ? acc + v[u] * b[u] : acc;" % (B // 16))
+    w.close()
+    w("acc += __shfl_xor(acc, 16);")
+    w("acc += __shfl_xor(acc, 32);")
+    w("if ((threadIdx.x & 63) < 16) s_part[(threadIdx.x >> 6) * 16 + q] = acc;")
+    w("__syncthreads();")
+    w.open("if (threadIdx.x < 16 && kc + q < khi)")
+    w("double t = s_part[q];")
+    w("for (int v = 1; v < %d; ++v) t += s_part[v * 16 + q];" % WAVES)
+    w("__builtin_nontemporal_store(t, %s + row * %s + k);" % (out_name, kext))
+    w.close()
+    w("__syncthreads();")
+    w.close()
+    w.close()
+    w.close()
+    w("return;")
+    w.close()
+    w("const tg_i64 row0 = (tg_i64)(blockIdx.x - n_help) * %d;" % TR)
+
+
+def _spmm_wave_calls(w: _W, low: Lowering, geo: LaunchGeometry, out_name: str, b_name: str,
+                     kext: str, V: int) -> None:
+    """A tile's row pointers in LDS, and the path its rows and K ask for; falls through to
+    the lane groups' rows."""
+    B, TR, U = geo.block, geo.rows_per_block, max(1, low.unroll)
+    WAVES = B // WAVE
+    LONG, HUGE, LH = 16 * U, 64 * U, spmm_huge(B, U)
+    w("// row pointers of this tile, its rows left to the helpers (s_huge) and whether it is")
+    w("// skewed")
+    w("__shared__ tg_i64 s_ptr[%d];" % (TR + 1))
+    w("__shared__ int s_huge[%d];" % (TR // 4 + 1))
+    w("__shared__ int s_nh;")
+    w("__shared__ tg_i64 s_col[2];")
+    w("__shared__ int s_skew;")
+    w("const tg_i64 t_rows = row_end - row0 < %d ? row_end - row0 : %d;" % (TR, TR))
+    w("if (threadIdx.x == 0) { s_nh = 0; s_skew = 0; }")
+    w("const tg_i64 rlast = row_end > 0 ? row_end : 0;")
+    w("tg_i64 pv = indptr[row0 + threadIdx.x < rlast ? row0 + threadIdx.x : rlast];")
+    w("// the first and the last column of the tile's first row, in flight over the staging")
+    w("tg_i64 cc = 0;")
+    w.open("if (threadIdx.x < 64)")
+    w("const tg_i64 pa = tg_lane_read(pv, 0), pb = tg_lane_read(pv, 1);")
+    w("if (threadIdx.x < 2 && pb > pa) cc = indices[threadIdx.x == 0 ? pa : pb - 1];")
+    w.close()
+    w("if (threadIdx.x <= %d) s_ptr[threadIdx.x] = pv;" % TR)
+    if TR + 1 > B:
+        w("#pragma unroll 1")
+        w.open("for (int t = threadIdx.x + %d; t <= %d; t += %d)" % (B, TR, B))
+        w("s_ptr[t] = indptr[row0 + t < rlast ? row0 + t : rlast];")
+        w.close()
+    w("__syncthreads();")
+    w("const tg_i64 t_nnz = s_ptr[%d] - s_ptr[0];" % TR)
+    w("#pragma unroll 1")
+    w.open("for (int t = threadIdx.x; t < t_rows; t += %d)" % B)
+    w("const tg_i64 n = s_ptr[t + 1] - s_ptr[t];")
+    w("if (n > %d && n * t_rows > 4 * t_nnz && n_help > 0) s_huge[atomicAdd(&s_nh, 1)] = t;" % LH)
+    w("if %s s_skew = 1;" % _long_row_test("n", LONG, HUGE))
+    w.close()
+    w("if (threadIdx.x < 2) s_col[threadIdx.x] = cc;")
+    w("__syncthreads();")
+    TPR, SLOTS = max(1, low.threads_per_row), B // max(1, low.threads_per_row)
+    # The rule's lines, each side measured (us a launch; 16 nonzeros per row over 100 k rows
+    # unless said otherwise, 16-row tiles on one wave; skewed matrices on 128-row tiles):
+    #   B rows of whole 128-byte lines: lane groups 98 / 217 at K = 64 / 128, one wave per
+    #     nonzero 117 / 235.  They pass over 16 columns (one line) at a time, so the tiles in
+    #     flight share a narrower stretch of B and 1 in 4 gathered lines hits L2; what is left
+    #     comes from the Infinity Cache at 6.9 TB/s, its rate for streams.
+    #   other K: a 16-column slice straddles two lines, which the next slice fetches again:
+    #     lane groups 190 / 340 / 534 at K = 33 / 63 / 130, one wave per nonzero (each line
+    #     once) 86 / 146 / 271, 7.2 TB/s at K = 130.  Up to 32 columns a wave would be half
+    #     empty: both slices of a nonzero at once, 114 -> 77 at K = 30, 73 -> 54 at K = 20.
+    #   columns close together (a band): B comes from L2 and the lane groups wait for their
+    #     index loads: one wave per nonzero 80 against 96 at K = 64, 137 against 196 at 128
+    #     (7 diagonals, 200 k rows).
+    #   skewed tiles: runs of equal length per wave and helpers for the dwarfing rows 114
+    #     against 353 (power law, K = 64), 92 against 315 (1% of rows 2000 long).
+    #   few waves: 2000 rows 9.7 against 15.4 at K = 64 and 9.9 against 18.2 at K = 33;
+    #     10000 rows (625 waves) 20.9 against 30.4.
+    w("const bool lines = ((%s & 15) == 0) && ((((unsigned long long)%s) & 127) == 0);"
+      % (kext, b_name))
+    w("// a grid of under 8 waves per CU waits for latency: two column slices and 3 nonzeros of")
+    w("// a row at a time")
+    w("const bool few = tn * %d < %d && %s <= 64;" % (WAVES, 8 * 256, kext))
+    w("bool wave = s_skew || (!lines && %s > 32 && !few);" % kext)
+    w("const tg_i64 span = tg_uniform(s_col[1] - s_col[0]);")
+    w("if (%s > 32 && !few && span < 256 && span > -256 && s_ptr[1] > s_ptr[0] + 1) wave = true;" % kext)
+    w.open("if (wave)")
+    w("if (t_rows <= 0) return;")
+    w("const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);")
+    w("const int nh = s_nh;")
+
+    def call(cl: int, e: int, u: int) -> str:
+        return ("tg_spmm_wave<%d, %d, %d, %d>(indices, data, %s, %s, %s, row0, (int)t_rows, s_ptr, "
+                "s_huge, nh, s_part, wv);" % (cl, e, u, WAVES, b_name, out_name, kext))
+    w("if (%s <= 64) %s" % (kext, call(1, 1, 16)))
+    w("else if (%s <= 128) %s" % (kext, call(2, 1, 8) if V == 2 else call(1, 2, 8)))
+    w("else %s" % (call(2, 2, 4) if V == 2 else call(1, 4, 4)))
+    w("return;")
+    w.close()
+    w.open("if (!lines || few)")
+    w("#pragma unroll 1")
+    w("for (tg_i64 kb = 0; kb < %s; kb += %d) tg_spmm_rows<%d, %d, 2, %d, %d>(indices, data, %s, "
+      "%s, %s, row0, (int)t_rows, s_ptr, kb);"
+      % (kext, 2 * TPR * V, TPR, V, 3, SLOTS, b_name, out_name, kext))
+    w("return;")
+    w.close()
+
+
 def _hip_row_dense_out(w: _W, plan: Plan, low: Lowering, bound: str, geo: LaunchGeometry,
-                       out_name: str, b_name: str, kext: str) -> None:
+                       out_name: str, b_name: str, kext: str, pre: _W) -> None:
     """C[row, :] = sum over nonzeros data[p] * B[col, :]; written once.
 
     Tiled variants balance long rows like SpMV does: a row longer than LONG
@@ -2431,7 +2976,6 @@ def _hip_row_dense_out(w: _W, plan: Plan, low: Lowering, bound: str, geo: Launch
     coop = low.tiled
     uniform = TPR == WAVE
     w("const tg_i64 row_end = %s;" % bound)
-    w("const tg_i64 row0 = (tg_i64)blockIdx.x * %d;" % TR)
     w("const int lane = threadIdx.x %% %d;" % TPR)
     if uniform:
         w("// a whole wave per row: row bounds and (column, value) pairs are wave-uniform")
@@ -2441,26 +2985,23 @@ def _hip_row_dense_out(w: _W, plan: Plan, low: Lowering, bound: str, geo: Launch
     if V == 2:
         w("const bool vec_ok = ((%s & 1) == 0) && ((((unsigned long long)%s) | "
           "((unsigned long long)%s)) & 15) == 0;" % (kext, b_name, out_name))
-    if coop:
-        w("__shared__ int s_long[%d];   // rows left to the whole workgroup" % TR)
-        w("__shared__ int s_nlong;")
-        w("__shared__ double s_part[%d];  // partial C-row slices, one per lane group" % (B * V))
-        _tile_stats(w, TR)
-    w("#pragma unroll 1")
-    w.open("for (int r = 0; r < %d; ++r)" % R)
-    w("const int lr = slot + r * %d;" % SLOTS)
-    w("const tg_i64 row = row0 + lr;")
-    w("if (lr >= %d || row >= row_end) break;" % TR)
-    if uniform:
-        w("const tg_i64 rs = tg_uniform(indptr[row]);")
-        w("const tg_i64 re = tg_uniform(indptr[row + 1]);")
-    else:
-        w("const tg_i64 rs = indptr[row];")
-        w("const tg_i64 re = indptr[row + 1];")
-    if coop:
-        w.open("if (%s)" % _long_row_test("re - rs", LONG, HUGE))
-        w("if (lane == 0) s_long[atomicAdd(&s_nlong, 1)] = lr;")
-        w("continue;")
+
+    def rows(ptr: str, listed: bool) -> None:
+        """The tile's rows, one per lane group; ``ptr`` formats a row pointer's source."""
+        w("#pragma unroll 1")
+        w.open("for (int r = 0; r < %d; ++r)" % R)
+        w("const int lr = slot + r * %d;" % SLOTS)
+        w("const tg_i64 row = row0 + lr;")
+        w("if (lr >= %d || row >= row_end) break;" % TR)
+        rs, re = (ptr % "", ptr % " + 1")
+        w("const tg_i64 rs = %s;" % ("tg_uniform(%s)" % rs if uniform else rs))
+        w("const tg_i64 re = %s;" % ("tg_uniform(%s)" % re if uniform else re))
+        if listed:
+            w.open("if (%s)" % _long_row_test("re - rs", LONG, HUGE))
+            w("if (lane == 0) s_long[atomicAdd(&s_nlong, 1)] = lr;")
+            w("continue;")
+            w.close()
+        both(kloop)
         w.close()
 
     def kloop(vec: bool) -> None:
@@ -2524,9 +3065,9 @@ def _hip_row_dense_out(w: _W, plan: Plan, low: Lowering, bound: str, geo: Launch
         else:
             emit(False)
 
-    both(kloop)
-    w.close()
     if not coop:
+        w("const tg_i64 row0 = (tg_i64)blockIdx.x * %d;" % TR)
+        rows("indptr[row%s]", False)
         return
 
     def wg_long(vec: bool) -> None:
@@ -2577,6 +3118,16 @@ def _hip_row_dense_out(w: _W, plan: Plan, low: Lowering, bound: str, geo: Launch
         w("__syncthreads();")
         w.close()
 
+    pre(_SPMM_WAVE.strip("\n"))
+    w("__shared__ double s_part[%d];  // partial C-row slices" % spmm_part(B, V))
+    w("// Up to %d columns: lane groups alone (the code of this path comes first, where a small" % SPMM_WAVE_K)
+    w("// launch fetches it soonest)")
+    w.open("if (%s <= %d)" % (kext, SPMM_WAVE_K))
+    w("const tg_i64 row0 = (tg_i64)blockIdx.x * %d;" % TR)
+    w("__shared__ int s_long[%d];   // rows left to the whole workgroup" % TR)
+    w("__shared__ int s_nlong;")
+    _tile_stats(w, TR)
+    rows("indptr[row%s]", True)
     w("// long rows: every lane group takes a strided share of the row's nonzeros")
     w("__syncthreads();")
     w("const int n_long = s_nlong;")
@@ -2586,6 +3137,11 @@ def _hip_row_dense_out(w: _W, plan: Plan, low: Lowering, bound: str, geo: Launch
     w("const tg_i64 crs = indptr[row], cre = indptr[row + 1];")
     both(wg_long)
     w.close()
+    w("return;")
+    w.close()
+    _spmm_helpers(w, plan, low, geo, out_name, b_name, kext)
+    _spmm_wave_calls(w, low, geo, out_name, b_name, kext, V)
+    rows("s_ptr[lr%s]", False)
 
 
 def _hip_sparse_out(w: _W, plan: Plan, low: Lowering, bound: str, geo: LaunchGeometry,
@@ -2882,7 +3438,8 @@ def _hip_kernel_text(kernel: Kernel, config: Config, plan: Plan, low: Lowering,
     out_name = plan.out_tensor.name
     pre = _W()  # file-scope declarations the kernel needs
     w = _W()
-    w("extern \"C\" __global__ __launch_bounds__(%d)" % geo.block)
+    w("extern \"C\" __global__ __launch_bounds__(%d)%s" % (
+        geo.block, " __attribute__((amdgpu_waves_per_eu(7)))" if geo.helper_div else ""))
     params = _hip_decls(args)
     if scratch_arg:
         params += ", unsigned long long* __restrict__ tg_part"
@@ -2895,7 +3452,7 @@ def _hip_kernel_text(kernel: Kernel, config: Config, plan: Plan, low: Lowering,
                            scratch_arg=scratch_arg)
     elif plan.kind == "row_dense_out":
         kext = _extent_for(plan, plan.inner_out[0].name)
-        _hip_row_dense_out(w, plan, low, bound, geo, out_name, _dense_name(plan, 0), kext)
+        _hip_row_dense_out(w, plan, low, bound, geo, out_name, _dense_name(plan, 0), kext, pre)
     elif plan.kind == "sparse_out":
         kext = _extent_for(plan, plan.reduce.index.name)
         _hip_sparse_out(w, plan, low, bound, geo, out_name, _dense_name(plan, 0),
@@ -2921,9 +3478,12 @@ def _check_hip_dtype(config: Config) -> None:
 def _grid_text(geo: LaunchGeometry) -> str:
     if geo.stream:
         return "floor(nnz / %d) + 1 (0 without rows)" % geo.nnz_chunk
-    return "ceil(%s / %d)%s" % (geo.rows_symbol, geo.rows_per_block,
-                                " + floor(nnz / %d) + 1" % geo.nnz_chunk if geo.nnz_chunk
-                                else "")
+    text = "ceil(%s / %d)" % (geo.rows_symbol, geo.rows_per_block)
+    if geo.nnz_chunk:
+        text += " + floor(nnz / %d) + 1" % geo.nnz_chunk
+    if geo.helper_div:
+        text += " + %d ceil(%s / hr)" % (SPMM_SLICES, geo.rows_symbol)
+    return text
 
 
 def emit_hip(kernel: Kernel, config: Config, scratch_arg: bool = False) -> str:
@@ -3056,7 +3616,16 @@ int tgv_launch_async(void* stream, %(params)s) {
         "extra": ("\n  /* long-row workgroups of hybrid tiles, ahead of the row tiles: one per"
                   "\n     range that nnz nonzeros can meet (ranges start at an even position) */"
                   "\n  if (*grid > 0) *grid += (nnz > 0 ? nnz : 0) / %d + 1;"
-                  % geo.nnz_chunk) if geo.nnz_chunk and not geo.stream else "",
+                  % geo.nnz_chunk) if geo.nnz_chunk and not geo.stream else
+                 ("\n  /* helper workgroups ahead of the tiles, for rows that dwarf their tile */"
+                  "\n  if (*grid > 0 && K > %d) {"
+                  "\n    int64_t hr = (rows / %d + 63) / 64 * 64;"
+                  "\n    hr = hr < 64 ? 64 : hr > %d ? %d : hr;"
+                  "\n    const int64_t help = %d * ((rows + hr - 1) / hr);"
+                  "\n    if ((*grid + help) * %d <= 0xFFFFFFFFLL) *grid += help;"
+                  "\n  }"
+                  % (SPMM_WAVE_K, geo.helper_div, SPMM_HELP_MAX, SPMM_HELP_MAX, SPMM_SLICES,
+                     geo.block)) if geo.helper_div else "",
     }
     return text
 
