@@ -33,7 +33,8 @@ backend "hip"
         u nonzeros' B rows in flight.  With k = 64 the row is wave-uniform and
         (column, value) pairs arrive through the scalar unit.  C is written
         exactly once per element (no read-modify-write), with nontemporal
-        stores since the kernel never reads it back.
+        stores since the kernel never reads it back.  Tiled variants take K
+        over 16 by the path their tile asks for (``_spmm_wave_calls``).
     sparse_out (sddmm)
         ThreadsPerRow(k) lanes split the K-long dot product of one nonzero,
         Vectorize(2) = 128-bit loads of U and V rows, Unroll(u) = u K-chunks
@@ -42,7 +43,8 @@ backend "hip"
         instruction), U[row, :] held in registers, column indices loaded k at
         a time and broadcast across the group, V gathers batched ahead of the
         FMAs, one coalesced nontemporal store per k outputs (U rows, read once,
-        are nontemporal loads too).  Otherwise one wave per row.
+        are nontemporal loads too).  Otherwise equal runs of nonzeros per
+        wave, or one wave per row where rows share columns in dense blocks.
     elementwise (axpy)
         one lane per element.
 
@@ -217,6 +219,7 @@ class LaunchGeometry:
     nnz_chunk: int = 0
     stream: bool = False
     helper_div: int = 0
+    helper_K: int = 0
 
     def grid(self, rows: int, nnz: int = 0, K: int = 64) -> int:
         if rows <= 0:
@@ -231,6 +234,12 @@ class LaunchGeometry:
             help_ = SPMM_SLICES * ((int(rows) + hr - 1) // hr)
             if (g + help_) * self.block <= 0xFFFFFFFF:
                 g += help_
+        if self.helper_K and K <= self.helper_K:
+            help_ = min(SDDMM_HELP, 1 << ((g | 4).bit_length() - 3))
+            if (g + help_) * self.block <= 0xFFFFFFFF:
+                g += help_
+        elif self.helper_K and K > self.helper_K:
+            g = max(g, min(SDDMM_RUN_GRID, max(0, int(nnz)) // (SDDMM_RUN * (self.block // WAVE))))
         return g
 
     def to_dict(self) -> Dict[str, Any]:
@@ -242,6 +251,8 @@ class LaunchGeometry:
             d["stream"] = True
         if self.helper_div:
             d["helper_div"] = self.helper_div
+        if self.helper_K:
+            d["helper_K"] = self.helper_K
         return d
 
 
@@ -760,7 +771,9 @@ def launch_geometry(plan: Plan, low: Lowering) -> LaunchGeometry:
     if plan.kind == "sparse_out":
         # the chunked and the wave-per-row paths each list their tile's long rows
         lists = [(4, rows), (4, 1), (8, 1)] if low.tiled else []
-        return LaunchGeometry(rows, B, _lds_total(lists + lists), plan.row_extent)
+        V = 2 if low.vector_width >= 2 else 1
+        return LaunchGeometry(rows, B, _lds_total(lists + lists), plan.row_extent,
+                              helper_K=tpr * V * max(1, low.unroll) if low.tiled else 0)
     if plan.kind == "row_dense_out":
         if not low.tiled:
             return LaunchGeometry(rows, B, 0, plan.row_extent)
@@ -818,6 +831,15 @@ def spmm_helper_div(block: int) -> int:
 
 
 SPMM_HELP_MAX = 1024
+
+# Tiled SDDMM's chunked path: at most this many helpers for the rows that dwarf their tile, on
+# ranges of at least SDDMM_HELP_MIN positions (powers of two)
+SDDMM_HELP = 512
+SDDMM_HELP_MIN = 256
+# Runs of nonzeros (K past the chunked path): a grid of few tiles grows to at most this many
+# workgroups, while their waves still take this many nonzeros each
+SDDMM_RUN_GRID = 1024
+SDDMM_RUN = 32
 
 
 def spmm_helper_rows(rows: int, div: int) -> int:
@@ -2464,7 +2486,7 @@ def _value_with(plan: Plan, data_text: str, gathered_text: str, row: str, col_te
     return rec(plan.value_expr)
 
 
-_SPMM_WAVE = r"""
+_LANE_COLS = r"""
 // Value of v held by lane src (uniform) of the wave.
 __device__ __forceinline__ tg_i64 tg_lane_read(tg_i64 v, int src) {
   const int lo = __builtin_amdgcn_readlane((int)v, src);
@@ -2486,7 +2508,9 @@ template <> struct tg_cols<2> {
   typedef double t __attribute__((ext_vector_type(2), aligned(8)));
   static __device__ __forceinline__ double get(t v, int c) { return c ? v.y : v.x; }
 };
+"""
 
+_SPMM_WAVE = r"""
 // Wave path of SpMM: the tile's nonzeros (but those of the rows listed in s_huge) are cut
 // into one equal run per wave, and a wave walks its run in position order with all 64 lanes
 // on one nonzero's B row: 64 CL E columns a pass, U nonzeros' loads in flight.  Column and
@@ -3118,6 +3142,7 @@ def _hip_row_dense_out(w: _W, plan: Plan, low: Lowering, bound: str, geo: Launch
         w("__syncthreads();")
         w.close()
 
+    pre(_LANE_COLS.strip("\n"))
     pre(_SPMM_WAVE.strip("\n"))
     w("__shared__ double s_part[%d];  // partial C-row slices" % spmm_part(B, V))
     w("// Up to %d columns: lane groups alone (the code of this path comes first, where a small" % SPMM_WAVE_K)
@@ -3145,13 +3170,13 @@ def _hip_row_dense_out(w: _W, plan: Plan, low: Lowering, bound: str, geo: Launch
 
 
 def _hip_sparse_out(w: _W, plan: Plan, low: Lowering, bound: str, geo: LaunchGeometry,
-                    out_name: str, u_name: str, v_name: str, kext: str) -> None:
+                    out_name: str, u_name: str, v_name: str, kext: str, pre: _W) -> None:
     """out[p] = data[p] * dot(U[row, :], V[col, :]) over the row's nonzeros.
 
     Two paths in one kernel, chosen by K at run time: the chunked path of
     ``_hip_sparse_out_fast`` when one lane group covers K with registers
-    (K <= TPR*V*U), else one wave per row with the lane groups spread over the
-    row's nonzeros and each group looping over K."""
+    (K <= TPR*V*U; for 128-bit loads also K even and both bases aligned), else
+    equal runs of nonzeros per wave (``_SDDMM_RUN``)."""
     B, TPR = geo.block, max(1, low.threads_per_row)
     U = max(1, low.unroll)
     V = 2 if low.vector_width >= 2 else 1
@@ -3159,8 +3184,24 @@ def _hip_sparse_out(w: _W, plan: Plan, low: Lowering, bound: str, geo: LaunchGeo
     SLOTS = WAVE // TPR
     TR = geo.rows_per_block
     R = (TR + WAVES - 1) // WAVES
+    env = _Env({plan.row_idx.name: "0"}, p="p", acc="res")
+    pre(_LANE_COLS.strip("\n"))
+    pre(_SDDMM_RUN.strip("\n").replace("TG_FINAL", _cexpr(plan.final_expr, env)))
     w("const tg_i64 row_end = %s;" % bound)
-    w("const tg_i64 row0 = (tg_i64)blockIdx.x * %d;" % TR)
+    if geo.helper_K:
+        w("// workgroups ahead of the tiles, one per 4 of them but at most %d, each at a boundary" % SDDMM_HELP)
+        w("// of ranges of ch positions (both powers of two: no division)")
+        w("const tg_i64 tn = (%s + %d) / %d;" % (plan.row_extent, TR - 1, TR))
+        w("int hs = 61 - __builtin_clzll((unsigned long long)(tn | 4));")
+        w("hs = hs < %d ? hs : %d;" % (SDDMM_HELP.bit_length() - 1, SDDMM_HELP.bit_length() - 1))
+        w("int n_help = %s <= %d ? 1 << hs : 0;" % (kext, geo.helper_K))
+        w("const tg_i64 per = nnz > 0 ? nnz >> hs : 0;")
+        w("const int chs = per < %d ? %d : 64 - __builtin_clzll((unsigned long long)per);"
+          % (SDDMM_HELP_MIN, SDDMM_HELP_MIN.bit_length() - 1))
+        w("if ((tn + n_help) * %d > 0xFFFFFFFFLL) n_help = 0;" % B)
+        w("const tg_i64 row0 = ((tg_i64)blockIdx.x - n_help) * %d;" % TR)
+    else:
+        w("const tg_i64 row0 = (tg_i64)blockIdx.x * %d;" % TR)
     w("const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / %d);" % WAVE)
     w("const int wl = threadIdx.x %% %d;" % WAVE)
     w("const int kq = wl %% %d;      // lane within the group" % TPR)
@@ -3171,7 +3212,29 @@ def _hip_sparse_out(w: _W, plan: Plan, low: Lowering, bound: str, geo: LaunchGeo
     _hip_sparse_out_fast(w, plan, TPR, U, V, SLOTS, WAVES, TR, out_name, u_name, v_name, kext,
                          coop=low.tiled)
     w.open("else")
+    w("if (row_end <= 0) return;")
+    w.open("if (%s <= 64 || !tg_blocked(indptr, indices, row_end))" % kext)
+    # over 64 columns (the runs' one nonzero per wave) a dense block's rows lose the V rows
+    # that neighbours share: 261 us by runs, 196 a row per wave side by side (4x4 blocks, 4 per
+    # row, K = 130); up to 64 the runs are ahead there too (63 against 119 at K = 33)
+    if V == 1:
+        forms = [(16, 16, 1, 1), (32, 32, 1, 1), (64, 64, 1, 1), (128, 64, 1, 2), (0, 64, 1, 4)]
+    else:
+        forms = [(16, 16, 1, 1), (32, 16, 2, 1), (64, 32, 2, 1), (128, 64, 2, 1), (0, 64, 2, 2)]
+    w("// equal runs of the launch's nonzeros per wave, whatever rows they lie in")
+    w("const tg_i64 gw = (tg_i64)blockIdx.x * %d + wave, nw = (tg_i64)gridDim.x * %d;"
+      % (WAVES, WAVES))
+    for n, (top, g, cl, e) in enumerate(forms):
+        w("%s%stg_sddmm_run<%d, %d, %d>(indptr, indices, data, %s, %s, %s, %s, row_end, gw, nw);"
+          % ("else " if n else "", "if (%s <= %d) " % (kext, top) if top else "", g, cl, e,
+             u_name, v_name, out_name, kext))
+    w("return;")
+    w.close()
+    w("// rows of dense blocks: a row per wave, the rows of a block side by side, so that they")
+    w("// gather the same V rows within a workgroup")
     coop = low.tiled
+    if coop:
+        w("if (row0 < 0) return;  // a helper of the chunked path")
     LONG = 8 * SLOTS   # 8 wave steps ...
     HUGE = 16 * SLOTS
 
@@ -3271,7 +3334,221 @@ def _hip_sparse_out(w: _W, plan: Plan, low: Lowering, bound: str, geo: LaunchGeo
         w("const tg_i64 re = tg_uniform(indptr[row + 1]);")
         row_body("rs + (tg_i64)wave * %d" % SLOTS, WAVES * SLOTS)
         w.close()
-    w.close()  # else (general path)
+    w.close()  # else
+
+
+_SDDMM_RUN = r"""
+// v in the lanes without BIT and w in those with it, each with the value of the lane across
+// BIT (its mirror where that is what DPP has) added: one halving step of a sum over lanes.
+template <int BIT>
+__device__ __forceinline__ double tg_halve(double v, double w) {
+  const bool hi = threadIdx.x & BIT;
+  const double mine = hi ? w : v, other = hi ? v : w;
+  return mine + (BIT >= 16 ? __shfl_xor(other, BIT) : BIT == 8 ? tg_dpp<0x140>(other)
+               : BIT == 4 ? tg_dpp<0x141>(other) : BIT == 2 ? tg_dpp<0x4E>(other)
+                                                            : tg_dpp<0xB1>(other));
+}
+// Sums of a[0..N-1] over each group of G lanes (N <= G): the lanes q of a group end with
+// the sum of a[q / (G / N)].  N - 1 halving steps and log2(G / N) whole ones, where N
+// butterflies would take N log2 G.
+template <int G, int N>
+__device__ __forceinline__ double tg_sums(const double* a) {
+  if constexpr (N == 1) {
+    return tg_segsum<G>(a[0]);
+  } else {
+    double b[N / 2];
+    #pragma unroll
+    for (int i = 0; i < N / 2; ++i) b[i] = tg_halve<G / 2>(a[i], a[i + N / 2]);
+    return tg_sums<G / 2, N / 2>(b);
+  }
+}
+
+// The row holding position P, pb = indptr[0] <= P < pe = indptr[R], and its bounds: 64
+// probes a round, the first of them the rows either side of the proportional guess, which
+// is all that rows of like length need.
+__device__ __forceinline__ tg_i64 tg_row_of(const tg_i64* __restrict__ indptr, const tg_i64 R,
+                                            const tg_i64 P, const tg_i64 pb, const tg_i64 pe,
+                                            tg_i64* rs, tg_i64* re) {
+  const int l = threadIdx.x & 63;
+  tg_i64 lo = 0, hi = R, vlo = pb, vhi = pe;   // indptr[lo] = vlo <= P < vhi = indptr[hi]
+  tg_i64 q = (tg_i64)((double)(P - pb) * ((double)R / (double)(pe - pb))) + l - 31;
+  #pragma unroll 1
+  for (;;) {
+    q = q < lo ? lo : (q > hi ? hi : q);
+    const tg_i64 v = indptr[q];
+    const unsigned long long m = __ballot(v > P);
+    const int f = m ? (int)__builtin_ctzll(m) : 64;   // first lane past P
+    if (f < 64) { hi = tg_lane_read(q, f); vhi = tg_lane_read(v, f); }
+    if (f > 0) { lo = tg_lane_read(q, f - 1); vlo = tg_lane_read(v, f - 1); }
+    if (hi - lo <= 1) break;
+    q = lo + 1 + (tg_i64)l * ((hi - lo + 61) / 63);
+  }
+  *rs = vlo;
+  *re = vhi;
+  return lo;
+}
+
+// Whether neighbouring rows mostly name the same columns (dense blocks): 16 pairs of rows
+// across the matrix, the same ones for every wave, at least 6 of which begin alike.
+__device__ __forceinline__ bool tg_blocked(const tg_i64* __restrict__ indptr,
+                                           const tg_i64* __restrict__ indices, const tg_i64 R) {
+  const int i = threadIdx.x & 63;
+  tg_i64 r = R * i / 16 + (i & 3);
+  const bool in = i < 16 && r + 2 <= R;
+  if (!in) r = 0;
+  const tg_i64 p0 = indptr[r], p1 = indptr[r + 1], p2 = indptr[in ? r + 2 : r + 1];
+  bool same = in && p1 > p0 && p2 > p1;
+  if (same) same = indices[p0] == indices[p1];
+  return __builtin_amdgcn_readfirstlane(__builtin_popcountll(__ballot(same))) >= 6;
+}
+
+// SDDMM by runs: wave gw of nw takes the positions [a, b), an equal share of the launch's
+// nonzeros, so that neither long rows nor many short ones leave waves idle.  G lanes take
+// one nonzero, CL E columns each of G CL E columns at a time; 8 nonzeros per group of G lanes
+// are in flight, and their dot products are summed over the lanes together (tg_sums).  Rows
+// and columns of 64 positions are kept one per lane.  Nonzeros of one row share the row's U
+// slice; where the batch spans rows each loads its own, which L1 holds.
+// Bound by the V gathers: 1.6 M nonzeros over 130 columns (uniform, 100 k rows) take 293 us,
+// 1.84 GB in lines from the Infinity Cache at 6.3 TB/s; a power law's 0.8 M take 163 where a
+// wave per row took 730 (its rows of 5000 on one workgroup), 55 against 444 at K = 33.  2 to 8
+// nonzeros' loads at once keep the kernel under 128 VGPRs, the chunked path's 4 waves per SIMD.
+template <int G, int CL, int E>
+__device__ __forceinline__ void tg_sddmm_run(
+    const tg_i64* __restrict__ indptr, const tg_i64* __restrict__ indices,
+    const double* __restrict__ data, const double* __restrict__ Um,
+    const double* __restrict__ Vm, double* __restrict__ out, const tg_i64 K, const tg_i64 R,
+    const tg_i64 gw, const tg_i64 nw) {
+  typedef typename tg_cols<CL>::t cols;
+  constexpr int NB = 8 * (64 / G);          // nonzeros per batch
+  constexpr int SH = G == 64 ? 3 : G == 32 ? 2 : 1;
+  constexpr int NC = G * CL * E;            // columns per pass
+  const tg_i64 pb = indptr[0], pe = indptr[R];
+  const tg_i64 len = ((pe - pb + nw - 1) / nw + NB - 1) / NB * NB;
+  const tg_i64 a = pb + gw * len;
+  const tg_i64 b = a + len < pe ? a + len : pe;
+  if (a >= b) return;
+  const int l = threadIdx.x & 63;
+  const int q = l & (G - 1), grp = l / G;
+  tg_i64 row0 = 0;                           // the row holding the chunk's first position
+  #pragma unroll 1
+  for (tg_i64 pc = a; pc < b; pc += 64) {
+    const int n = (int)(b - pc < 64 ? b - pc : 64);
+    const tg_i64 jl = indices[pc + (l < n ? l : n - 1)];
+    tg_i64 r0, r1;
+    if (pc == a) row0 = tg_row_of(indptr, R, pc, pb, pe, &r0, &r1);
+    // the rows of the chunk's positions: the ends of 64 rows from row0 on, searched by each
+    // lane; where rows without nonzeros use those up, a new search for the first lane left
+    tg_i64 rl = -1;
+    tg_i64 base = row0;
+    #pragma unroll 1
+    for (;;) {
+      const tg_i64 re = indptr[base + 1 + l < R ? base + 1 + l : R] - pc;
+      const int end = re < 127 ? (int)re : 127;
+      int c = 0;                              // row ends at or before position l
+      #pragma unroll
+      for (int d = 32; d; d >>= 1) {
+        const int e = __shfl(end, c + d - 1);
+        if (e <= l) c += d;
+      }
+      const int e = __shfl(end, 63);
+      if (rl < 0 && !(c == 63 && e <= l)) rl = base + c;
+      const unsigned long long left = __ballot(rl < 0 && l < n);
+      if (!left) break;
+      base = tg_row_of(indptr, R, pc + (int)__builtin_ctzll(left), pb, pe, &r0, &r1);
+    }
+    if (rl < 0) rl = row0;                    // lanes past the run
+    #pragma unroll 1
+    for (int s = 0; s < n; s += NB) {
+      const int last = s + NB < n ? s + NB - 1 : n - 1;
+      const tg_i64 rf = tg_lane_read(rl, s);
+      const bool one = tg_lane_read(rl, last) == rf;
+      double acc[8];
+      #pragma unroll
+      for (int u = 0; u < 8; ++u) acc[u] = 0.0;
+      #pragma unroll 1
+      for (tg_i64 kb = 0; kb < K; kb += NC) {
+        const tg_i64 kbase = kb >= 2 ? kb - 2 : 0;
+        const int left = K - kb < NC ? (int)(K - kb) : NC;   // columns of this pass
+        unsigned ko[E];
+        #pragma unroll
+        for (int e = 0; e < E; ++e) {
+          const int k = e * G * CL + q * CL;
+          ko[e] = (unsigned)((k + CL <= left ? k : left - CL) + (int)(kb - kbase)) * 8u;
+        }
+        // a slice of columns: whole (every lane's count), partly past K or all past K
+        auto fma = [&](double& t, int e, const cols& x, const cols& y) {
+          if ((e + 1) * G * CL <= left) {
+            #pragma unroll
+            for (int c = 0; c < CL; ++c) t += tg_cols<CL>::get(x, c) * tg_cols<CL>::get(y, c);
+          } else {
+            const int k = e * G * CL + q * CL;
+            #pragma unroll
+            for (int c = 0; c < CL; ++c)
+              t = (c == CL - 1 ? k < left : k + CL <= left)
+                  ? t + tg_cols<CL>::get(x, c) * tg_cols<CL>::get(y, c) : t;
+          }
+        };
+        const char* const Vk = (const char*)(Vm + kbase);
+        const char* const Uk = (const char*)(Um + kbase);
+        if (one) {
+          cols ur[E];
+          #pragma unroll
+          for (int e = 0; e < E; ++e) ur[e] = *(const cols*)(Uk + rf * K * 8 + ko[e]);
+          constexpr int H = E == 1 ? 8 : 4;   // at once: 8 of the widest form pass 128 VGPRs
+          #pragma unroll
+          for (int h = 0; h < 8; h += H) {
+            cols v[H][E];
+            #pragma unroll
+            for (int u = 0; u < H; ++u) {
+              int t = s + grp * 8 + h + u;
+              t = t < n ? t : n - 1;
+              const tg_i64 j = G == 64 ? tg_lane_read(jl, t) : tg_lane_bcast(jl, t);
+              #pragma unroll
+              for (int e = 0; e < E; ++e) v[u][e] = *(const cols*)(Vk + j * K * 8 + ko[e]);
+            }
+            #pragma unroll
+            for (int u = 0; u < H; ++u)
+              #pragma unroll
+              for (int e = 0; e < E; ++e)
+                if (e * G * CL < left) fma(acc[h + u], e, ur[e], v[u][e]);
+          }
+        } else {
+          constexpr int H = E == 1 ? 4 : 2;
+          #pragma unroll
+          for (int h = 0; h < 8; h += H) {
+            cols x[H][E], v[H][E];
+            #pragma unroll
+            for (int u = 0; u < H; ++u) {
+              int t = s + grp * 8 + h + u;
+              t = t < n ? t : n - 1;
+              const tg_i64 j = G == 64 ? tg_lane_read(jl, t) : tg_lane_bcast(jl, t);
+              const tg_i64 r = G == 64 ? tg_lane_read(rl, t) : tg_lane_bcast(rl, t);
+              #pragma unroll
+              for (int e = 0; e < E; ++e) {
+                v[u][e] = *(const cols*)(Vk + j * K * 8 + ko[e]);
+                x[u][e] = *(const cols*)(Uk + r * K * 8 + ko[e]);
+              }
+            }
+            #pragma unroll
+            for (int u = 0; u < H; ++u)
+              #pragma unroll
+              for (int e = 0; e < E; ++e)
+                if (e * G * CL < left) fma(acc[h + u], e, x[u][e], v[u][e]);
+            __builtin_amdgcn_sched_barrier(0);   // this part's registers before the next's loads
+          }
+        }
+      }
+      const double res = tg_sums<G, 8>(acc);
+      const int t = s + (l >> SH);
+      if (t < n && (l & ((1 << SH) - 1)) == 0) {
+        const tg_i64 p = pc + t;
+        __builtin_nontemporal_store(TG_FINAL, out + p);
+      }
+    }
+    row0 = tg_lane_read(rl, n - 1);
+  }
+}
+"""
 
 
 def _sddmm_batch(TPR: int, E: int) -> int:
@@ -3298,8 +3575,9 @@ def _hip_sparse_out_fast(w: _W, plan: Plan, TPR: int, U: int, V: int, SLOTS: int
     coalesced store.  With ``coop`` (tiled variants) a row longer than 8
     chunks is listed in LDS instead, and after the tile's other rows every
     lane group of the workgroup takes a strided share of its chunks (SDDMM
-    outputs need no reduction across nonzeros).  Opens an ``if``; the caller
-    emits the general path in the matching ``else``."""
+    outputs need no reduction across nonzeros); a row that dwarfs its tile
+    goes to the helper workgroups ahead of the tiles.  Opens an ``if``; the caller
+    emits the other paths in the matching ``else``."""
     W = V
     KCAP = TPR * V * U
     E = U * W
@@ -3335,16 +3613,18 @@ def _hip_sparse_out_fast(w: _W, plan: Plan, TPR: int, U: int, V: int, SLOTS: int
         w("const tg_i64 jl = mine ? indices[rs + q + kq] : 0;")
         w("const double dl = mine ? data[rs + q + kq] : 0.0;")
         w("double res = 0.0;")
+        w("// batch b: nonzeros b, b + %d, ... of the chunk, so that lane kq's sum is nonzero kq's"
+          % (TPR // NB))
         w("#pragma unroll")
-        w.open("for (int n0 = 0; n0 < %d; n0 += %d)" % (TPR, NB))
-        w("double x[%d][%d];" % (NB, E))
+        w.open("for (int b = 0; b < %d; ++b)" % (TPR // NB))
+        w("double x[%d][%d], acc[%d];" % (NB, E, NB))
         w("#pragma unroll")
         w.open("for (int n = 0; n < %d; ++n)" % NB)
         if TPR > 1:
-            w("const tg_i64 j = tg_lane_bcast(jl, slot * %d + n0 + n);" % TPR)
+            w("const tg_i64 j = tg_lane_bcast(jl, slot * %d + n * %d + b);" % (TPR, TPR // NB))
         else:
             w("const tg_i64 j = jl;")
-        w("const bool v = q + n0 + n < len;")
+        w("const bool v = q + n * %d + b < len;" % (TPR // NB))
         w("const double* __restrict__ vr = %s + j * %s;" % (v_name, kext))
         w("#pragma unroll")
         w.open("for (int u = 0; u < %d; ++u)" % U)
@@ -3361,13 +3641,12 @@ def _hip_sparse_out_fast(w: _W, plan: Plan, TPR: int, U: int, V: int, SLOTS: int
         w.close()
         w("#pragma unroll")
         w.open("for (int n = 0; n < %d; ++n)" % NB)
-        w("double acc = 0.0;")
+        w("acc[n] = 0.0;")
         w("#pragma unroll")
-        w("for (int e = 0; e < %d; ++e) acc += ur[e] * x[n][e];" % E)
-        if TPR > 1:
-            w("acc = tg_segsum<%d>(acc);" % TPR)
-        w("if (kq == n0 + n) res = acc;")
+        w("for (int e = 0; e < %d; ++e) acc[n] += ur[e] * x[n][e];" % E)
         w.close()
+        w("const double sum = tg_sums<%d, %d>(acc);" % (TPR, NB))
+        w("if (%s) res = sum;" % ("kq %% %d == b" % (TPR // NB) if TPR > NB else "true"))
         w.close()
         env = _Env({plan.row_idx.name: "row"}, p="(rs + q + kq)", acc="res", data="dl")
         w("if (mine) __builtin_nontemporal_store(%s, %s + rs + q + kq);"
@@ -3378,6 +3657,28 @@ def _hip_sparse_out_fast(w: _W, plan: Plan, TPR: int, U: int, V: int, SLOTS: int
     w("// one lane group per row; chunks of %d nonzeros, V slices gathered %d at a time"
       % (TPR, NB))
     if coop:
+        w.open("if (row0 < 0)")
+        w("// Helper e: when the row that holds position e ch dwarfs its tile, that row's positions")
+        w("// from there to the next boundary, and those before it when this is the row's first.")
+        w("// On a power law (100 k rows, 800 k nonzeros) 512 of them take K = 64 from 147 to 95 us")
+        w("// (256: 119, 128: 145) and K = 8 from 120 to 68; rows of like length cost them one")
+        w("// probe of the row pointers, 0.3 us of 26 at K = 8")
+        w("const tg_i64 ch = 1LL << chs, P = (tg_i64)blockIdx.x << chs;")
+        w("if (row_end <= 0) return;")
+        w("const tg_i64 pb = tg_uniform(indptr[0]), pe = tg_uniform(indptr[row_end]);")
+        w("if (P < pb || P >= pe) return;")
+        w("tg_i64 r0, r1;")
+        w("const tg_i64 row = tg_row_of(indptr, row_end, P, pb, pe, &r0, &r1);")
+        w("if (r1 - r0 <= ch || r1 - r0 <= %d || r1 > (tg_i64)n_help << chs) return;" % LONG)
+        w("const tg_i64 t0 = row / %d * %d, t1 = t0 + %d < row_end ? t0 + %d : row_end;"
+          % (TR, TR, TR, TR))
+        w("if ((r1 - r0) * (t1 - t0) <= 4 * (indptr[t1] - indptr[t0])) return;")
+        w("const tg_i64 rs = P - ch < r0 ? r0 : P;")
+        w("const tg_i64 len = (P + ch < r1 ? P + ch : r1) - rs;")
+        load_u("true")
+        chunks("(tg_i64)(wave * %d + slot) * %d" % (SLOTS, TPR), B)
+        w("return;")
+        w.close()
         w("__shared__ int s_long[%d];   // rows left to the whole workgroup" % TR)
         w("__shared__ int s_nlong;")
         _tile_stats(w, TR)
@@ -3390,7 +3691,10 @@ def _hip_sparse_out_fast(w: _W, plan: Plan, TPR: int, U: int, V: int, SLOTS: int
     if coop:
         w("tg_i64 len = live ? indptr[row + 1] - rs : 0;")
         w.open("if (%s)" % _long_row_test("len", LONG, HUGE))
-        w("if (kq == 0) s_long[atomicAdd(&s_nlong, 1)] = lr;")
+        w("// (a row that dwarfs the tile and holds a helper's boundary is the helpers')")
+        w("const bool away = len > (1LL << chs) && len * t_rows > 4 * t_nnz "
+          "&& rs + len <= (tg_i64)n_help << chs;")
+        w("if (kq == 0 && !away) s_long[atomicAdd(&s_nlong, 1)] = lr;")
         w("len = 0;  // the lane group skips it")
         w.close()
     else:
@@ -3439,7 +3743,8 @@ def _hip_kernel_text(kernel: Kernel, config: Config, plan: Plan, low: Lowering,
     pre = _W()  # file-scope declarations the kernel needs
     w = _W()
     w("extern \"C\" __global__ __launch_bounds__(%d)%s" % (
-        geo.block, " __attribute__((amdgpu_waves_per_eu(7)))" if geo.helper_div else ""))
+        geo.block, " __attribute__((amdgpu_waves_per_eu(%d)))" % (7 if geo.helper_div else 4)
+        if plan.kind == "row_dense_out" and low.tiled else ""))
     params = _hip_decls(args)
     if scratch_arg:
         params += ", unsigned long long* __restrict__ tg_part"
@@ -3456,7 +3761,7 @@ def _hip_kernel_text(kernel: Kernel, config: Config, plan: Plan, low: Lowering,
     elif plan.kind == "sparse_out":
         kext = _extent_for(plan, plan.reduce.index.name)
         _hip_sparse_out(w, plan, low, bound, geo, out_name, _dense_name(plan, 0),
-                        _dense_name(plan, 1), kext)
+                        _dense_name(plan, 1), kext, pre)
     elif plan.kind == "elementwise":
         _hip_elementwise(w, plan, bound, geo, out_name)
     else:  # pragma: no cover
@@ -3483,6 +3788,8 @@ def _grid_text(geo: LaunchGeometry) -> str:
         text += " + floor(nnz / %d) + 1" % geo.nnz_chunk
     if geo.helper_div:
         text += " + %d ceil(%s / hr)" % (SPMM_SLICES, geo.rows_symbol)
+    if geo.helper_K:
+        text += " + helpers"
     return text
 
 
@@ -3625,7 +3932,21 @@ int tgv_launch_async(void* stream, %(params)s) {
                   "\n    if ((*grid + help) * %d <= 0xFFFFFFFFLL) *grid += help;"
                   "\n  }"
                   % (SPMM_WAVE_K, geo.helper_div, SPMM_HELP_MAX, SPMM_HELP_MAX, SPMM_SLICES,
-                     geo.block)) if geo.helper_div else "",
+                     geo.block)) if geo.helper_div else
+                 ("\n  /* helper workgroups ahead of the tiles, for rows that dwarf their tile */"
+                  "\n  if (*grid > 0 && K <= %d) {"
+                  "\n    int hs = 61 - __builtin_clzll((unsigned long long)(*grid | 4));"
+                  "\n    const int64_t help = (int64_t)1 << (hs < %d ? hs : %d);"
+                  "\n    if ((*grid + help) * %d <= 0xFFFFFFFFLL) *grid += help;"
+                  "\n  } else if (*grid > 0 && K > %d) {"
+                  "\n    /* runs of nonzeros: enough workgroups for a wave to each %d of few rows */"
+                  "\n    const int64_t runs = nnz / %d < %d ? nnz / %d : %d;"
+                  "\n    if (*grid < runs) *grid = runs;"
+                  "\n  }"
+                  % (geo.helper_K, SDDMM_HELP.bit_length() - 1, SDDMM_HELP.bit_length() - 1,
+                     geo.block, geo.helper_K, SDDMM_RUN, SDDMM_RUN * (geo.block // WAVE),
+                     SDDMM_RUN_GRID, SDDMM_RUN * (geo.block // WAVE), SDDMM_RUN_GRID))
+                 if geo.helper_K else "",
     }
     return text
 
