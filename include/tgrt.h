@@ -82,7 +82,7 @@ int tg_launch(tg_function fn, int64_t grid, int32_t block, int32_t lds_bytes,
 
 /* tg_launch, ordered after the previous launch made with the same order_key on
  * the current device: when that launch went to another stream, `stream` first
- * waits for its end (an event recorded after every such launch).  Generated
+ * waits for its end (an event attached to every such launch).  Generated
  * launchers of kernels that combine row pieces through module scratch pass
  * their embedded code object as the key, so calls that overlap on two streams
  * run one after the other instead of racing on the scratch.  A launch into a
