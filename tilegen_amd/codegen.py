@@ -782,8 +782,11 @@ def launch_geometry(plan: Plan, low: Lowering) -> LaunchGeometry:
         # dwarfing rows and their counts, the skew flag, the helpers' row bits, partial C-row slices
         arrays = [(8, rows + 1), (8, 2), (8, 1), (4, rows), (4, 1), (4, rows // 4 + 1), (4, 1),
                   (4, 1), (8, SPMM_HELP_MAX // 64), (8, spmm_part(B, V))]
-        return LaunchGeometry(rows, B, _lds_total(arrays), plan.row_extent,
-                            helper_div=spmm_helper_div(B))
+        geo = LaunchGeometry(rows, B, 0, plan.row_extent, helper_div=spmm_helper_div(B))
+        if spmm_band(geo):
+            arrays += [(8, 16 * SPMM_BAND)]
+        geo.lds_bytes = _lds_total(arrays)
+        return geo
     if plan.kind != "scalar_reduce" or not low.tiled:
         return LaunchGeometry(rows, B, 0, plan.row_extent)
     if low.balance == "stream":
@@ -831,6 +834,17 @@ def spmm_helper_div(block: int) -> int:
 
 
 SPMM_HELP_MAX = 1024
+
+# SpMM's band path: B rows staged in LDS, 16 columns of them (3 KB: with the 1.4 KB of the
+# other paths a CU still holds 28 one-wave workgroups, as many as its registers allow)
+SPMM_BAND = 24
+
+
+def spmm_band(geo: "LaunchGeometry") -> bool:
+    """Tiles of one wave and up to 16 rows (a tile of more spans more B rows than are
+    staged) have the band path."""
+    return geo.block == WAVE and 8 <= geo.rows_per_block <= 16
+
 
 # Tiled SDDMM's chunked path: at most this many helpers for the rows that dwarf their tile, on
 # ranges of at least SDDMM_HELP_MIN positions (powers of two)
@@ -2752,6 +2766,141 @@ __device__ __forceinline__ void tg_spmm_wave(
   }
 }
 
+// Band path of SpMM, one wave per tile of up to 8 P rows: where no row has more than 8
+// nonzeros and the tile's columns lie within SPAN, the SPAN B rows are staged in LDS, 16
+// columns at a time, and every nonzero reads them there, so that a B row leaves L2 once per
+// tile and not once per nonzero.  8 lanes take a row, two columns each; lane u of them holds
+// the row's u-th nonzero, which ds_swizzle hands to the other 7.  The next 16 columns are
+// loaded while these are summed.  Rows are summed in position order.  False, with nothing
+// written, where the tile is no such band.
+// Bound by its streams: 7 diagonals, 200 k rows, against one wave per nonzero: K = 45 56.8 ->
+// 43.5 us, K = 64 59.8 -> 44.6 (5.0 TB/s of B, C and the matrix), K = 128 113 -> 102; 100 k
+// rows, K = 256 170 -> 98; 50 k rows, K = 33 21.2 -> 14.0.  K = 130, cold: 169 -> 164.  C goes
+// through L2, which puts together the lines that two slices write in part: past the caches
+// K = 45 takes 66 us and K = 130 173, though whole lines would gain (K = 128 75).
+template <int P, int SPAN>
+__device__ __forceinline__ bool tg_spmm_band(
+    const tg_i64* __restrict__ indices, const double* __restrict__ data,
+    const double* __restrict__ Bm, double* __restrict__ C, const tg_i64 K, const tg_i64 row0,
+    const int nrows, const tg_i64* s_ptr, double* s_band) {
+  typedef typename tg_cols<2>::t cols;
+  const int q = threadIdx.x & 7, g = (threadIdx.x & 63) >> 3;
+  tg_i64 jmin = 0x7FFFFFFFFFFFFFFFll, jmax = -1;
+  int len[P], off[P];
+  tg_i64 j[P];
+  double v[P];
+  bool ok = true;
+  #pragma unroll
+  for (int p = 0; p < P; ++p) {
+    const int row = g + 8 * p;
+    const tg_i64 rs = s_ptr[row < nrows ? row : 0];
+    const tg_i64 n = row < nrows ? s_ptr[row + 1] - rs : 0;
+    ok &= n <= 8;
+    len[p] = (int)(n < 8 ? n : 8);
+    j[p] = 0;
+    v[p] = 0.0;
+    if (q < len[p]) {
+      j[p] = indices[rs + q];
+      v[p] = data[rs + q];
+    }
+  }
+  if (__ballot(!ok)) return false;
+  #pragma unroll
+  for (int p = 0; p < P; ++p) {
+    if (q < len[p]) {
+      jmin = j[p] < jmin ? j[p] : jmin;
+      jmax = j[p] > jmax ? j[p] : jmax;
+    }
+  }
+  #pragma unroll
+  for (int d = 1; d < 64; d *= 2) {
+    const tg_i64 a = __shfl_xor(jmin, d), b = __shfl_xor(jmax, d);
+    jmin = a < jmin ? a : jmin;
+    jmax = b > jmax ? b : jmax;
+  }
+  jmin = tg_uniform(jmin);
+  jmax = tg_uniform(jmax);
+  if (jmax < jmin || jmax - jmin >= SPAN) return false;
+  const int ns = (int)(jmax - jmin) + 1;
+  #pragma unroll
+  for (int p = 0; p < P; ++p)   // bit 15: there is a nonzero
+    off[p] = q < len[p] ? (int)(j[p] - jmin) * 16 | 0x8000 : 0;
+  constexpr int NL = (SPAN + 7) / 8;
+  const char* const Bj = (const char*)(Bm + jmin * K);
+  const unsigned rk = (unsigned)K * 8u;
+  // this lane's i-th B row; past the span, the last one again
+  int gl = g;
+  auto brow = [&](int i) { return (unsigned)(gl + 8 * i < ns ? gl + 8 * i : ns - 1) * rk; };
+  cols t[NL];
+  // a lane past the last columns loads the last pair again
+  const int Kc = (int)K;
+  int k = 2 * q;
+  int kl = k <= Kc - 2 ? k : Kc - 2;
+  #pragma unroll
+  for (int i = 0; i < NL; ++i)
+    if (8 * i < ns) t[i] = *(const cols*)(Bj + (brow(i) + (unsigned)kl * 8u));
+  #pragma unroll 1
+  for (int kb = 0; kb < Kc; kb += 16) {
+    asm volatile("" : "+v"(gl));   // addresses made anew each time: kept, they spill
+    #pragma unroll
+    for (int i = 0; i < NL; ++i)
+      if (8 * i < ns && g + 8 * i < SPAN) {
+        s_band[(g + 8 * i) * 16 + 2 * q] = t[i].x;
+        s_band[(g + 8 * i) * 16 + 2 * q + 1] = t[i].y;
+      }
+    __syncthreads();
+    const int kc = k;
+    k += 16;
+    kl = k <= Kc - 2 ? k : Kc - 2;
+    if (kb + 16 < Kc) {
+      #pragma unroll
+      for (int i = 0; i < NL; ++i)
+        if (8 * i < ns) t[i] = *(const cols*)(Bj + (brow(i) + (unsigned)kl * 8u));
+    }
+    #pragma unroll
+    for (int p = 0; p < P; ++p) {
+      double a0 = 0.0, a1 = 0.0;
+      const int vlo = (int)__double_as_longlong(v[p]);
+      const int vhi = (int)(__double_as_longlong(v[p]) >> 32);
+#define TG_BAND_STEP(u) \
+      { \
+        const int o = __builtin_amdgcn_ds_swizzle(off[p], (u << 5) | 0x18); \
+        const unsigned lo = (unsigned)__builtin_amdgcn_ds_swizzle(vlo, (u << 5) | 0x18); \
+        const int hi = __builtin_amdgcn_ds_swizzle(vhi, (u << 5) | 0x18); \
+        const double d = __longlong_as_double(((tg_i64)hi << 32) | (tg_i64)lo); \
+        const double* const b = s_band + ((o & 0x7FFF) + 2 * q); \
+        const double b0 = b[0], b1 = b[1]; \
+        a0 = o & 0x8000 ? a0 + d * b0 : a0; \
+        a1 = o & 0x8000 ? a1 + d * b1 : a1; \
+      }
+      __builtin_amdgcn_sched_barrier(0);   // two steps in flight: more spill (72 registers)
+      TG_BAND_STEP(0) TG_BAND_STEP(1)
+      __builtin_amdgcn_sched_barrier(0);
+      TG_BAND_STEP(2) TG_BAND_STEP(3)
+      __builtin_amdgcn_sched_barrier(0);
+      TG_BAND_STEP(4) TG_BAND_STEP(5)
+      __builtin_amdgcn_sched_barrier(0);
+      TG_BAND_STEP(6) TG_BAND_STEP(7)
+      __builtin_amdgcn_sched_barrier(0);
+#undef TG_BAND_STEP
+      const int row = g + 8 * p;
+      if (row < nrows && kc < Kc) {
+        double* const c = (double*)((char*)(C + row0 * K) + (unsigned)row * rk);
+        if (kc <= Kc - 2) {
+          cols o;
+          o.x = a0;
+          o.y = a1;
+          *(cols*)(c + kc) = o;
+        } else {
+          c[K - 1] = a1;   // odd K: the pair's second column is the last
+        }
+      }
+    }
+    __syncthreads();   // the next columns overwrite s_band
+  }
+  return true;
+}
+
 // Lane groups of SpMM: TPR lanes per row, CL E columns each from column kb on, the tile's
 // rows SLOTS apart, U nonzeros' B rows in flight.
 template <int TPR, int CL, int E, int U, int SLOTS>
@@ -2901,7 +3050,16 @@ def _spmm_helpers(w: _W, plan: Plan, low: Lowering, geo: LaunchGeometry, out_nam
     w.close()
     w("return;")
     w.close()
-    w("const tg_i64 row0 = (tg_i64)(blockIdx.x - n_help) * %d;" % TR)
+    if not spmm_band(geo):
+        w("const tg_i64 row0 = (tg_i64)(blockIdx.x - n_help) * %d;" % TR)
+        return
+    w("// Workgroups go to the 8 XCDs in turn.  Where rows have 8 nonzeros or fewer on average, as")
+    w("// the band path's do, each XCD takes a contiguous eighth of the tiles, so that a band's")
+    w("// neighbouring tiles share its L2: 7 diagonals, 200 k rows, K = 45 52.8 -> 42.6 us, K = 64")
+    w("// 49.2 -> 44.4.  100 k rows of 16 uniform columns, K = 64, take 101 us so and 98 in turn.")
+    w("const unsigned tb = blockIdx.x - n_help, xq = tn / 8, xr = tn % 8, xc = tb % 8;")
+    w("const tg_i64 row0 = (tg_i64)(nnz <= 8 * %s ? xc * xq + (xc < xr ? xc : xr) + tb / 8 : tb) * %d;"
+      % (plan.row_extent, TR))
 
 
 def _spmm_wave_calls(w: _W, low: Lowering, geo: LaunchGeometry, out_name: str, b_name: str,
@@ -2918,6 +3076,8 @@ def _spmm_wave_calls(w: _W, low: Lowering, geo: LaunchGeometry, out_name: str, b
     w("__shared__ int s_nh;")
     w("__shared__ tg_i64 s_col[2];")
     w("__shared__ int s_skew;")
+    if spmm_band(geo):
+        w("__shared__ double s_band[%d];" % (16 * SPMM_BAND))
     w("const tg_i64 t_rows = row_end - row0 < %d ? row_end - row0 : %d;" % (TR, TR))
     w("if (threadIdx.x == 0) { s_nh = 0; s_skew = 0; }")
     w("const tg_i64 rlast = row_end > 0 ? row_end : 0;")
@@ -2969,9 +3129,15 @@ def _spmm_wave_calls(w: _W, low: Lowering, geo: LaunchGeometry, out_name: str, b
     w("const bool few = tn * %d < %d && %s <= 64;" % (WAVES, 8 * 256, kext))
     w("bool wave = s_skew || (!lines && %s > 32 && !few);" % kext)
     w("const tg_i64 span = tg_uniform(s_col[1] - s_col[0]);")
-    w("if (%s > 32 && !few && span < 256 && span > -256 && s_ptr[1] > s_ptr[0] + 1) wave = true;" % kext)
+    w("const bool near = %s > 32 && !few && span < 256 && span > -256 && s_ptr[1] > s_ptr[0] + 1;"
+      % kext)
+    w("wave = wave || near;")
     w.open("if (wave)")
     w("if (t_rows <= 0) return;")
+    if spmm_band(geo):
+        w("if (near && !s_skew && %s <= (1 << 20) && tg_spmm_band<%d, %d>(indices, data, %s, %s, %s, "
+          "row0, (int)t_rows, s_ptr, s_band)) return;"
+          % (kext, (TR + 7) // 8, SPMM_BAND, b_name, out_name, kext))
     w("const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);")
     w("const int nh = s_nh;")
 
