@@ -466,6 +466,15 @@ def _extent_for(plan: Plan, index_name: str) -> str:
     return "K"
 
 
+def _dense_extent(plan: Plan) -> str:
+    """The extent of the dense index of a row_dense_out or sparse_out kernel ("K" for others)."""
+    if plan.kind == "row_dense_out":
+        return _extent_for(plan, plan.inner_out[0].name)
+    if plan.kind == "sparse_out":
+        return _extent_for(plan, plan.reduce.index.name)
+    return "K"
+
+
 class _W:
     """Indented line writer."""
 
@@ -2981,7 +2990,8 @@ def _spmm_helpers(w: _W, plan: Plan, low: Lowering, geo: LaunchGeometry, out_nam
          SPMM_HELP_MAX))
     w("hr = hr < 64 ? 64 : hr;")
     w("unsigned n_help = (unsigned)((%s + hr - 1) / hr) * %d;" % (plan.row_extent, NS))
-    w("if (((tg_i64)tn + n_help) * %d > 0xFFFFFFFFLL) n_help = 0;  // past one launch's work-items" % B)
+    w("// none past one launch's work-items, or where the caller's grid is for the tiles alone")
+    w("if (gridDim.x != tn + n_help) n_help = 0;")
     w("__shared__ unsigned long long s_hrow[%d];  // a helper's rows, one bit each" % (SPMM_HELP_MAX // 64))
     w.open("if (blockIdx.x < n_help)")
     w("// Helper: of its hr rows, those over %d nonzeros and over 4 times their tile's" % LH)
@@ -3377,7 +3387,8 @@ def _hip_sparse_out(w: _W, plan: Plan, low: Lowering, bound: str, geo: LaunchGeo
         w("const tg_i64 per = nnz > 0 ? nnz >> hs : 0;")
         w("const int chs = per < %d ? %d : 64 - __builtin_clzll((unsigned long long)per);"
           % (SDDMM_HELP_MIN, SDDMM_HELP_MIN.bit_length() - 1))
-        w("if ((tn + n_help) * %d > 0xFFFFFFFFLL) n_help = 0;" % B)
+        w("// none past one launch's work-items, or where the caller's grid is for the tiles alone")
+        w("if (gridDim.x != tn + n_help) n_help = 0;")
         w("const tg_i64 row0 = ((tg_i64)blockIdx.x - n_help) * %d;" % TR)
     else:
         w("const tg_i64 row0 = (tg_i64)blockIdx.x * %d;" % TR)
@@ -3935,10 +3946,10 @@ def _hip_kernel_text(kernel: Kernel, config: Config, plan: Plan, low: Lowering,
         _hip_scalar_reduce(w, plan, low, bound, geo, out_name, pre=pre,
                            scratch_arg=scratch_arg)
     elif plan.kind == "row_dense_out":
-        kext = _extent_for(plan, plan.inner_out[0].name)
+        kext = _dense_extent(plan)
         _hip_row_dense_out(w, plan, low, bound, geo, out_name, _dense_name(plan, 0), kext, pre)
     elif plan.kind == "sparse_out":
-        kext = _extent_for(plan, plan.reduce.index.name)
+        kext = _dense_extent(plan)
         _hip_sparse_out(w, plan, low, bound, geo, out_name, _dense_name(plan, 0),
                         _dense_name(plan, 1), kext, pre)
     elif plan.kind == "elementwise":
@@ -4026,7 +4037,9 @@ def emit_hip_host(kernel: Kernel, config: Config) -> str:
         else:
             pack.append("  a[%d] = (uint64_t)%s;" % (len(pack), n))
     uses_scratch = module_scratch(plan, low)
-    kdim = "K" if "K" in dims else "0"
+    # the grid counts helper workgroups by the dense extent the kernel compares, whatever its name
+    kext = _dense_extent(plan)
+    kdim = kext if kext in dims else "0"
     ndim = "N" if "N" in dims else "0"
     nnz = "nnz" if "nnz" in dims else "0"
     params = ", ".join("%s %s" % a for a in args)
