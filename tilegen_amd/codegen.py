@@ -63,6 +63,7 @@ from __future__ import annotations
 
 import hashlib
 import os
+import re
 from dataclasses import dataclass, field
 from typing import Any, Callable, Dict, List, Optional, Sequence, Tuple
 
@@ -3373,23 +3374,26 @@ def _hip_sparse_out(w: _W, plan: Plan, low: Lowering, bound: str, geo: LaunchGeo
     SLOTS = WAVE // TPR
     TR = geo.rows_per_block
     R = (TR + WAVES - 1) // WAVES
-    env = _Env({plan.row_idx.name: "0"}, p="p", acc="res")
+    # the output of position p in row ``row`` with the dot product res, as the runs call it; the
+    # row is handed over only where the expression reads it
+    final = _cexpr(plan.final_expr, _Env({plan.row_idx.name: "row"}, p="p", acc="res"))
     pre(_LANE_COLS.strip("\n"))
-    pre(_SDDMM_RUN.strip("\n").replace("TG_FINAL", _cexpr(plan.final_expr, env)))
+    pre(_SDDMM_RUN.strip("\n").replace(
+        "TG_ROW", "tg_lane_bcast(rl, t)" if re.search(r"\brow\b", final) else "0"))
     w("const tg_i64 row_end = %s;" % bound)
     if geo.helper_K:
         w("// workgroups ahead of the tiles, one per 4 of them but at most %d, each at a boundary" % SDDMM_HELP)
         w("// of ranges of ch positions (both powers of two: no division)")
-        w("const tg_i64 tn = (%s + %d) / %d;" % (plan.row_extent, TR - 1, TR))
-        w("int hs = 61 - __builtin_clzll((unsigned long long)(tn | 4));")
-        w("hs = hs < %d ? hs : %d;" % (SDDMM_HELP.bit_length() - 1, SDDMM_HELP.bit_length() - 1))
-        w("int n_help = %s <= %d ? 1 << hs : 0;" % (kext, geo.helper_K))
-        w("const tg_i64 per = nnz > 0 ? nnz >> hs : 0;")
-        w("const int chs = per < %d ? %d : 64 - __builtin_clzll((unsigned long long)per);"
+        w("const tg_i64 tg_tn = (%s + %d) / %d;" % (plan.row_extent, TR - 1, TR))
+        w("int tg_hs = 61 - __builtin_clzll((unsigned long long)(tg_tn | 4));")
+        w("tg_hs = tg_hs < %d ? tg_hs : %d;" % (SDDMM_HELP.bit_length() - 1, SDDMM_HELP.bit_length() - 1))
+        w("int tg_n_help = %s <= %d ? 1 << tg_hs : 0;" % (kext, geo.helper_K))
+        w("const tg_i64 tg_per = nnz > 0 ? nnz >> tg_hs : 0;")
+        w("const int tg_chs = tg_per < %d ? %d : 64 - __builtin_clzll((unsigned long long)tg_per);"
           % (SDDMM_HELP_MIN, SDDMM_HELP_MIN.bit_length() - 1))
         w("// none past one launch's work-items, or where the caller's grid is for the tiles alone")
-        w("if (gridDim.x != tn + n_help) n_help = 0;")
-        w("const tg_i64 row0 = ((tg_i64)blockIdx.x - n_help) * %d;" % TR)
+        w("if (gridDim.x != tg_tn + tg_n_help) tg_n_help = 0;")
+        w("const tg_i64 row0 = ((tg_i64)blockIdx.x - tg_n_help) * %d;" % TR)
     else:
         w("const tg_i64 row0 = (tg_i64)blockIdx.x * %d;" % TR)
     w("const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / %d);" % WAVE)
@@ -3412,11 +3416,14 @@ def _hip_sparse_out(w: _W, plan: Plan, low: Lowering, bound: str, geo: LaunchGeo
     else:
         forms = [(16, 16, 1, 1), (32, 16, 2, 1), (64, 32, 2, 1), (128, 64, 2, 1), (0, 64, 2, 2)]
     w("// equal runs of the launch's nonzeros per wave, whatever rows they lie in")
-    w("const tg_i64 gw = (tg_i64)blockIdx.x * %d + wave, nw = (tg_i64)gridDim.x * %d;"
+    w("const tg_i64 tg_gw = (tg_i64)blockIdx.x * %d + wave, tg_nw = (tg_i64)gridDim.x * %d;"
       % (WAVES, WAVES))
+    w("const auto tg_final = [&](const tg_i64 p, const tg_i64 row, const double res) -> double {")
+    w("  return %s;" % final)
+    w("};")
     for n, (top, g, cl, e) in enumerate(forms):
-        w("%s%stg_sddmm_run<%d, %d, %d>(indptr, indices, data, %s, %s, %s, %s, row_end, gw, nw);"
-          % ("else " if n else "", "if (%s <= %d) " % (kext, top) if top else "", g, cl, e,
+        w("%s%stg_sddmm_run<%d, %d, %d>(indptr, indices, data, %s, %s, %s, %s, row_end, tg_gw, "
+          "tg_nw, tg_final);" % ("else " if n else "", "if (%s <= %d) " % (kext, top) if top else "", g, cl, e,
              u_name, v_name, out_name, kext))
     w("return;")
     w.close()
@@ -3602,12 +3609,12 @@ __device__ __forceinline__ bool tg_blocked(const tg_i64* __restrict__ indptr,
 // 1.84 GB in lines from the Infinity Cache at 6.3 TB/s; a power law's 0.8 M take 163 where a
 // wave per row took 730 (its rows of 5000 on one workgroup), 55 against 444 at K = 33.  2 to 8
 // nonzeros' loads at once keep the kernel under 128 VGPRs, the chunked path's 4 waves per SIMD.
-template <int G, int CL, int E>
+template <int G, int CL, int E, class F>
 __device__ __forceinline__ void tg_sddmm_run(
     const tg_i64* __restrict__ indptr, const tg_i64* __restrict__ indices,
     const double* __restrict__ data, const double* __restrict__ Um,
     const double* __restrict__ Vm, double* __restrict__ out, const tg_i64 K, const tg_i64 R,
-    const tg_i64 gw, const tg_i64 nw) {
+    const tg_i64 gw, const tg_i64 nw, const F final) {
   typedef typename tg_cols<CL>::t cols;
   constexpr int NB = 8 * (64 / G);          // nonzeros per batch
   constexpr int SH = G == 64 ? 3 : G == 32 ? 2 : 1;
@@ -3730,9 +3737,10 @@ __device__ __forceinline__ void tg_sddmm_run(
       }
       const double res = tg_sums<G, 8>(acc);
       const int t = s + (l >> SH);
+      const tg_i64 row = TG_ROW;
       if (t < n && (l & ((1 << SH) - 1)) == 0) {
         const tg_i64 p = pc + t;
-        __builtin_nontemporal_store(TG_FINAL, out + p);
+        __builtin_nontemporal_store(final(p, row, res), out + p);
       }
     }
     row0 = tg_lane_read(rl, n - 1);
@@ -3853,18 +3861,18 @@ def _hip_sparse_out_fast(w: _W, plan: Plan, TPR: int, U: int, V: int, SLOTS: int
         w("// On a power law (100 k rows, 800 k nonzeros) 512 of them take K = 64 from 147 to 95 us")
         w("// (256: 119, 128: 145) and K = 8 from 120 to 68; rows of like length cost them one")
         w("// probe of the row pointers, 0.3 us of 26 at K = 8")
-        w("const tg_i64 ch = 1LL << chs, P = (tg_i64)blockIdx.x << chs;")
+        w("const tg_i64 tg_ch = 1LL << tg_chs, tg_P = (tg_i64)blockIdx.x << tg_chs;")
         w("if (row_end <= 0) return;")
-        w("const tg_i64 pb = tg_uniform(indptr[0]), pe = tg_uniform(indptr[row_end]);")
-        w("if (P < pb || P >= pe) return;")
-        w("tg_i64 r0, r1;")
-        w("const tg_i64 row = tg_row_of(indptr, row_end, P, pb, pe, &r0, &r1);")
-        w("if (r1 - r0 <= ch || r1 - r0 <= %d || r1 > (tg_i64)n_help << chs) return;" % LONG)
-        w("const tg_i64 t0 = row / %d * %d, t1 = t0 + %d < row_end ? t0 + %d : row_end;"
+        w("const tg_i64 tg_pb = tg_uniform(indptr[0]), tg_pe = tg_uniform(indptr[row_end]);")
+        w("if (tg_P < tg_pb || tg_P >= tg_pe) return;")
+        w("tg_i64 tg_r0, tg_r1;")
+        w("const tg_i64 row = tg_row_of(indptr, row_end, tg_P, tg_pb, tg_pe, &tg_r0, &tg_r1);")
+        w("if (tg_r1 - tg_r0 <= tg_ch || tg_r1 - tg_r0 <= %d || tg_r1 > (tg_i64)tg_n_help << tg_chs) return;" % LONG)
+        w("const tg_i64 tg_t0 = row / %d * %d, tg_t1 = tg_t0 + %d < row_end ? tg_t0 + %d : row_end;"
           % (TR, TR, TR, TR))
-        w("if ((r1 - r0) * (t1 - t0) <= 4 * (indptr[t1] - indptr[t0])) return;")
-        w("const tg_i64 rs = P - ch < r0 ? r0 : P;")
-        w("const tg_i64 len = (P + ch < r1 ? P + ch : r1) - rs;")
+        w("if ((tg_r1 - tg_r0) * (tg_t1 - tg_t0) <= 4 * (indptr[tg_t1] - indptr[tg_t0])) return;")
+        w("const tg_i64 rs = tg_P - tg_ch < tg_r0 ? tg_r0 : tg_P;")
+        w("const tg_i64 len = (tg_P + tg_ch < tg_r1 ? tg_P + tg_ch : tg_r1) - rs;")
         load_u("true")
         chunks("(tg_i64)(wave * %d + slot) * %d" % (SLOTS, TPR), B)
         w("return;")
@@ -3882,8 +3890,8 @@ def _hip_sparse_out_fast(w: _W, plan: Plan, TPR: int, U: int, V: int, SLOTS: int
         w("tg_i64 len = live ? indptr[row + 1] - rs : 0;")
         w.open("if (%s)" % _long_row_test("len", LONG, HUGE))
         w("// (a row that dwarfs the tile and holds a helper's boundary is the helpers')")
-        w("const bool away = len > (1LL << chs) && len * t_rows > 4 * t_nnz "
-          "&& rs + len <= (tg_i64)n_help << chs;")
+        w("const bool away = len > (1LL << tg_chs) && len * t_rows > 4 * t_nnz "
+          "&& rs + len <= (tg_i64)tg_n_help << tg_chs;")
         w("if (kq == 0 && !away) s_long[atomicAdd(&s_nlong, 1)] = lr;")
         w("len = 0;  // the lane group skips it")
         w.close()
