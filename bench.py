@@ -228,7 +228,7 @@ class CaseRun:
         self.K = self.case.K
         self.ops = baseline_operands(self.kernel, self.M, self.N, self.K)
         self.v = Variant(self.kernel, cfg)
-        self.fn = self.v.function()
+        self.fn = self.v.function(self.K)
         self.grid, self.block, self.lds = self.v.geometry(self.M, self.N, self.K, self.nnz)
         self.nbytes = compulsory_bytes(self.kernel, self.M, self.N, self.nnz, self.K)
         self.nflop = flops(self.kernel, self.nnz, self.K)

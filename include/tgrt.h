@@ -64,6 +64,12 @@ int tg_module_function(tg_module module, const char* name, tg_function* fn);
  * once per (code pointer, device) and kept until tg_code_release. */
 int tg_code_function(const void* code, size_t code_size, const char* name,
                      tg_function* fn);
+
+/* The same for a library that embeds two code objects with a kernel of one name: the
+ * call that loads `code` also loads `other` and looks its kernel up, so that no later
+ * call has to (a stream may be capturing by then). */
+int tg_code_function_beside(const void* code, size_t code_size, const void* other,
+                            size_t other_size, const char* name, tg_function* fn);
 /* Forgets the cached modules of an embedded code object on every device, so
  * that another object later placed at the same address is loaded afresh.
  * Generated launcher libraries call it as they are unloaded.  The modules are

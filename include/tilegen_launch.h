@@ -77,6 +77,10 @@ void launch_axpy(const double* x, const double* w, double* z, double alpha, doub
 
 /* Harness side of a variant library (no counterpart in the reference). */
 void* tgv_function(void);                  /* the variant's kernel, current device */
+/* the kernel that a launch with K dense columns takes where its operands are 16-byte
+ * aligned: SpMM and SDDMM have one of few columns in a code object of its own;
+ * tgv_function's is right at any K */
+void* tgv_function_for(int64_t K);
 const char* tgv_kernel_name(void);         /* "spmv", "spmm", ... */
 /* grid and block of a launch; *lds_bytes is the dynamic LDS to pass, always 0:
  * every generated kernel declares its LDS statically */

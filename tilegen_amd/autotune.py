@@ -288,7 +288,8 @@ def _make_caller(lib_path: str, kernel_name: str, A: sp.csr_matrix, data, K: int
     fn.argtypes = _SIGNATURES[kernel_name]
     if backend == "hip":
         from . import runtime as rt
-        lib.tgv_function.restype = ctypes.c_void_p
+        lib.tgv_function_for.restype = ctypes.c_void_p
+        lib.tgv_function_for.argtypes = [ctypes.c_int64]
         lib.tgv_geometry.argtypes = [ctypes.c_int64] * 4 + [
             ctypes.POINTER(ctypes.c_int64), ctypes.POINTER(ctypes.c_int32),
             ctypes.POINTER(ctypes.c_int32)]
@@ -308,9 +309,9 @@ def _make_caller(lib_path: str, kernel_name: str, A: sp.csr_matrix, data, K: int
 
         def timer(warmup: int, iters: int) -> np.ndarray:
             rt.lib().tg_clear_error()
-            kfn = lib.tgv_function()
+            kfn = lib.tgv_function_for(Kd)
             if not kfn:
-                rt.check_status("tgv_function")
+                rt.check_status("tgv_function_for")
             if geom[0] == 0:
                 return np.zeros(iters)
             kms, _wall = rt.time_launches(kfn, geom[0], geom[1], geom[2], bench.sets,

@@ -866,6 +866,17 @@ SDDMM_RUN_GRID = 1024
 SDDMM_RUN = 32
 
 
+def spmm_waves(low: Lowering) -> int:
+    """Waves per SIMD asked of the compiler for the kernel of K over SPMM_WAVE_K, 0 for none.
+    Seven (72 registers) where the schedule's own batch of B rows, unroll x vector width, leaves
+    room for it: c4's lane groups take 98 us at 7 and 122 at 6, 4-lane groups of unroll 4 265 and
+    275, 16-lane groups of width 1 132 and 139 (uniform, K = 64).  A batch of 16 doubles spills
+    8 registers at 7 (131 us against 116 at 6, 32-lane groups of unroll 8), one of 32 spills at
+    any request."""
+    batch = max(1, low.unroll) * (2 if low.vector_width >= 2 else 1)
+    return 7 if batch <= 8 else 6 if batch <= 16 else 0
+
+
 def spmm_helper_rows(rows: int, div: int) -> int:
     """Rows whose pointers one helper scans, whole 64-lane ballots of them."""
     return min(SPMM_HELP_MAX, max(64, (rows // div + 63) // 64 * 64))
@@ -877,16 +888,15 @@ def spmm_huge(block: int, unroll: int) -> int:
     return max(2 * block, 16 * unroll)
 
 
-def spmm_cols(V: int) -> int:
-    """Columns per pass of the wave path's widest form: 64 lanes, four each."""
-    return 256
+# columns per pass of the wave path's widest form: 64 lanes, four each
+SPMM_COLS = 256
 
 
 def spmm_part(block: int, V: int) -> int:
     """Doubles of the partial C-row slices: one slice per lane group, or two rows'
     pieces per wave on the wave path."""
     waves = block // WAVE
-    return max(block * V, 2 * waves * spmm_cols(V) if waves > 1 else 0)
+    return max(block * V, 2 * waves * SPMM_COLS if waves > 1 else 0)
 
 
 # Stream ranges: at most this many nonzeros per workgroup (their products are
@@ -2557,8 +2567,10 @@ _SPMM_WAVE = r"""
 // began before the run, slot 1: of the row that runs past its end) and the wave the row ends
 // in adds them in wave order after one barrier.
 // Bound by gathers: 1.6 M nonzeros over 130 columns take 271 us, 1.95 GB in lines from the
-// Infinity Cache; 4 to 16 nonzeros in flight per wave keep the kernel at 72 VGPRs, 7 waves
-// per SIMD, which the lane groups' paths need more than this one does (98 us at 7, 122 at 6).
+// Infinity Cache; 4 to 16 nonzeros in flight per wave fit the 72 VGPRs that the kernel is held
+// to for the lane groups' sake (spmm_waves).  Pairs of columns need 8-byte alignment only, so
+// schedules without 128-bit loads take the same forms: half the loads, and no spill where the
+// forms of single columns left 3 to 13 registers in scratch.
 template <int CL, int E, int U, int WAVES>
 __device__ __forceinline__ void tg_spmm_wave(
     const tg_i64* __restrict__ indices, const double* __restrict__ data,
@@ -3156,8 +3168,8 @@ def _spmm_wave_calls(w: _W, low: Lowering, geo: LaunchGeometry, out_name: str, b
         return ("tg_spmm_wave<%d, %d, %d, %d>(indices, data, %s, %s, %s, row0, (int)t_rows, s_ptr, "
                 "s_huge, nh, s_part, wv);" % (cl, e, u, WAVES, b_name, out_name, kext))
     w("if (%s <= 64) %s" % (kext, call(1, 1, 16)))
-    w("else if (%s <= 128) %s" % (kext, call(2, 1, 8) if V == 2 else call(1, 2, 8)))
-    w("else %s" % (call(2, 2, 4) if V == 2 else call(1, 4, 4)))
+    w("else if (%s <= 128) %s" % (kext, call(2, 1, 8)))
+    w("else %s" % call(2, 2, 4))
     w("return;")
     w.close()
     w.open("if (!lines || few)")
@@ -3337,7 +3349,7 @@ def _hip_row_dense_out(w: _W, plan: Plan, low: Lowering, bound: str, geo: Launch
     w("__shared__ double s_part[%d];  // partial C-row slices" % spmm_part(B, V))
     w("// Up to %d columns: lane groups alone (the code of this path comes first, where a small" % SPMM_WAVE_K)
     w("// launch fetches it soonest)")
-    w.open("if (%s <= %d)" % (kext, SPMM_WAVE_K))
+    w.open("if (SMALL || %s <= %d)" % (kext, SPMM_WAVE_K))
     w("const tg_i64 row0 = (tg_i64)blockIdx.x * %d;" % TR)
     w("__shared__ int s_long[%d];   // rows left to the whole workgroup" % TR)
     w("__shared__ int s_nlong;")
@@ -3354,9 +3366,11 @@ def _hip_row_dense_out(w: _W, plan: Plan, low: Lowering, bound: str, geo: Launch
     w.close()
     w("return;")
     w.close()
+    w.open("if constexpr (!SMALL)")
     _spmm_helpers(w, plan, low, geo, out_name, b_name, kext)
     _spmm_wave_calls(w, low, geo, out_name, b_name, kext, V)
     rows("s_ptr[lr%s]", False)
+    w.close()
 
 
 def _hip_sparse_out(w: _W, plan: Plan, low: Lowering, bound: str, geo: LaunchGeometry,
@@ -3405,7 +3419,7 @@ def _hip_sparse_out(w: _W, plan: Plan, low: Lowering, bound: str, geo: LaunchGeo
           "((unsigned long long)%s)) & 15) == 0;" % (kext, u_name, v_name))
     _hip_sparse_out_fast(w, plan, TPR, U, V, SLOTS, WAVES, TR, out_name, u_name, v_name, kext,
                          coop=low.tiled)
-    w.open("else")
+    w.open("else if constexpr (!SMALL)")
     w("if (row_end <= 0) return;")
     w.open("if (%s <= 64 || !tg_blocked(indptr, indices, row_end))" % kext)
     # over 64 columns (the runs' one nonzero per wave) a dense block's rows lose the V rows
@@ -3851,7 +3865,7 @@ def _hip_sparse_out_fast(w: _W, plan: Plan, TPR: int, U: int, V: int, SLOTS: int
           % (_cexpr(plan.final_expr, env), out_name))
         w.close()
 
-    w.open("if (%s)" % cond)
+    w.open("if (SMALL || (%s))" % cond)
     w("// one lane group per row; chunks of %d nonzeros, V slices gathered %d at a time"
       % (TPR, NB))
     if coop:
@@ -3940,12 +3954,24 @@ def _hip_kernel_text(kernel: Kernel, config: Config, plan: Plan, low: Lowering,
     out_name = plan.out_tensor.name
     pre = _W()  # file-scope declarations the kernel needs
     w = _W()
-    w("extern \"C\" __global__ __launch_bounds__(%d)%s" % (
-        geo.block, " __attribute__((amdgpu_waves_per_eu(%d)))" % (7 if geo.helper_div else 4)
-        if plan.kind == "row_dense_out" and low.tiled else ""))
     params = _hip_decls(args)
     if scratch_arg:
         params += ", unsigned long long* __restrict__ tg_part"
+    bounds = "extern \"C\" __global__ __launch_bounds__(%d)" % geo.block
+    if small_kernel_test(plan, low):
+        # two code objects of one text: the whole kernel, and the path of few columns alone,
+        # which needs far fewer registers than the others and would share their occupancy
+        waves = spmm_waves(low) if plan.kind == "row_dense_out" else 0
+        w("#ifdef TG_SMALL")
+        w("constexpr bool SMALL = true;")
+        w("#define TG_WAVES")
+        w("#else")
+        w("constexpr bool SMALL = false;")
+        w("#define TG_WAVES%s" % (" __attribute__((amdgpu_waves_per_eu(%d)))" % waves if waves
+                                  else ""))
+        w("#endif")
+        bounds += " TG_WAVES"
+    w(bounds)
     w.open("void %s_kernel(%s)" % (kernel.name, params))
     if plan.kind == "scalar_reduce":
         if not plan.reduce_is_compressed:
@@ -3966,6 +3992,24 @@ def _hip_kernel_text(kernel: Kernel, config: Config, plan: Plan, low: Lowering,
         raise NotImplementedError(plan.kind)
     w.close()
     return pre.text() + ("\n" if pre.lines else "") + w.text()
+
+
+def small_kernel_test(plan: Plan, low: Lowering) -> str:
+    """C condition on a launch's arguments for the code object compiled with TG_SMALL, the
+    kernel's path of few columns alone, or "" where a variant has one code object.  Every launch
+    the condition admits takes the same path in the whole kernel, which is right for all."""
+    kext = _dense_extent(plan)
+    if plan.kind == "row_dense_out" and low.tiled:
+        return "%s <= %d" % (kext, SPMM_WAVE_K)
+    if plan.kind == "sparse_out":
+        V = 2 if low.vector_width >= 2 else 1
+        cap = "%s <= %d" % (kext, max(1, low.threads_per_row) * V * max(1, low.unroll))
+        if V == 1:
+            return cap
+        u, v = _dense_name(plan, 0), _dense_name(plan, 1)
+        return ("%s && (%s & 1) == 0 && ((((unsigned long long)%s) | ((unsigned long long)%s)) & 15)"
+                " == 0" % (cap, kext, u, v))
+    return ""
 
 
 def _check_hip_dtype(config: Config) -> None:
@@ -4020,7 +4064,8 @@ def emit_hip_host(kernel: Kernel, config: Config) -> str:
     """C launcher for a HIP variant.
 
     ``{CODE_OBJECT}`` and ``{CODE_SIZE}`` are replaced by the compiled bytes
-    when the variant is built.  The launcher exports the reference ABI
+    when the variant is built (``{SMALL_OBJECT}`` and ``{SMALL_SIZE}`` by those compiled with
+    TG_SMALL, where ``small_kernel_test`` gives the launches that take them).  The launcher exports the reference ABI
     (synchronous, device pointers, errors reported through ``tg_last_error``)
     plus ``tgv_geometry``, ``tgv_function`` and ``tgv_launch_async`` for
     harnesses that time the kernel on their own stream.  Variants that combine
@@ -4051,26 +4096,51 @@ def emit_hip_host(kernel: Kernel, config: Config) -> str:
     ndim = "N" if "N" in dims else "0"
     nnz = "nnz" if "nnz" in dims else "0"
     params = ", ".join("%s %s" % a for a in args)
+    small = small_kernel_test(plan, low)
+    if small:
+        small_code = ("\n/* the path of few columns alone, in fewer registers */"
+                      "\nstatic const unsigned char tg_small[{SMALL_SIZE}] = {{SMALL_OBJECT}};")
+        pick = """/* either code object's first use loads both, so that a program which has launched
+   at one K can capture a launch at another */
+static void* tgv_pick(int small) {
+  tg_function fn = 0;
+  const int rc = small ? tg_code_function_beside(tg_small, sizeof(tg_small), tg_code,
+                                                 sizeof(tg_code), "%s", &fn)
+                       : tg_code_function_beside(tg_code, sizeof(tg_code), tg_small,
+                                                 sizeof(tg_small), "%s", &fn);
+  return rc == 0 ? fn : 0;
+}
+
+void* tgv_function(void) { return tgv_pick(0); }
+
+void* tgv_function_for(int64_t K) { return tgv_pick(%s); }
+""" % (sym, sym, small.split(" && ((((")[0].replace(kext, "K"))  # K of aligned operands
+        fn = "tgv_pick(%s)" % small
+    else:
+        small_code, fn = "", "tgv_function()"
+        pick = """void* tgv_function(void) {
+  tg_function fn = 0;
+  if (tg_code_function(tg_code, sizeof(tg_code), "%s", &fn) != 0) return 0;
+  return fn;
+}
+
+void* tgv_function_for(int64_t K) { (void)K; return tgv_function(); }
+""" % sym
     text = """/* TileGen HIP launcher for %(sym)s -- generated, DO NOT EDIT.
  * schedule %(sched)s; grid = %(grid_text)s, block = %(block)d, static lds = %(lds)d B */
 #include <stdint.h>
 #include <string.h>
 #include "tgrt.h"
 
-static const unsigned char tg_code[{CODE_SIZE}] = {{CODE_OBJECT}};
+static const unsigned char tg_code[{CODE_SIZE}] = {{CODE_OBJECT}};%(small_code)s
 
 /* the runtime caches the loaded module by tg_code's address: drop that entry
    when this library is unloaded, before another can be mapped there */
 __attribute__((destructor)) static void tgv_unload(void) {
-  tg_code_release(tg_code, sizeof(tg_code));
+  tg_code_release(tg_code, sizeof(tg_code));%(release)s
 }
 
-void* tgv_function(void) {
-  tg_function fn = 0;
-  if (tg_code_function(tg_code, sizeof(tg_code), "%(sym)s", &fn) != 0) return 0;
-  return fn;
-}
-
+%(pick)s
 const char* tgv_kernel_name(void) { return "%(name)s"; }
 
 int tgv_geometry(int64_t M, int64_t N, int64_t K, int64_t nnz,
@@ -4091,7 +4161,7 @@ static int tgv_pack(uint64_t* a, %(params)s) {
 }
 
 int tgv_launch_async(void* stream, %(params)s) {
-  tg_function fn = (tg_function)tgv_function();
+  tg_function fn = (tg_function)%(fn)s;
   if (!fn) return tg_last_status();
   int64_t grid; int32_t block, lds;
   tgv_geometry(%(M)s, %(N)s, %(K)s, %(nnz)s, &grid, &block, &lds);
@@ -4105,6 +4175,8 @@ int tgv_launch_async(void* stream, %(params)s) {
   if (tgv_launch_async(0, %(names)s) == 0) tg_synchronize();
 }
 """ % {
+        "pick": pick, "fn": fn, "small_code": small_code,
+        "release": "\n  tg_code_release(tg_small, sizeof(tg_small));" if small else "",
         "sym": sym, "name": kernel.name, "sched": config.short(), "rows": rows,
         "rpb": geo.rows_per_block, "block": geo.block, "lds": geo.lds_bytes,
         "rows_expr": rows if rows in dims else "M", "params": params,

@@ -288,15 +288,15 @@ int main(int argc, char** argv) {
   std::vector<float> kms;
   double enqueue_async_us = -1.0, enqueue_raw_us = -1.0;
   if (hip) {
-    using Fn = void* (*)(void);
+    using Fn = void* (*)(int64_t);
     using Fg = int (*)(int64_t, int64_t, int64_t, int64_t, int64_t*, int32_t*, int32_t*);
-    Fn getfn = reinterpret_cast<Fn>(dlsym(h, "tgv_function"));
+    Fn getfn = reinterpret_cast<Fn>(dlsym(h, "tgv_function_for"));
     Fg geom = reinterpret_cast<Fg>(dlsym(h, "tgv_geometry"));
     if (getfn && geom) {
       int64_t grid = 0;
       int32_t block = 0, lds = 0;
       geom(M, N, K, nnz, &grid, &block, &lds);
-      void* kfn = getfn();
+      void* kfn = getfn(K);
       if (kfn && grid > 0) {
         std::vector<uint64_t> slots;
         for (const Set& s : sets) {

@@ -242,19 +242,16 @@ int tg_module_function(tg_module module, const char* name, tg_function* fn) {
   return 0;
 }
 
-int tg_code_function(const void* code, size_t code_size, const char* name,
-                     tg_function* fn) {
-  if (!code || !code_size || !name || !fn) return fail(-1, "tg_code_function: null argument");
-  int device = 0;
-  TG_HIP(hipGetDevice(&device), "hipGetDevice");
-  CodeCache& c = code_cache();
-  std::lock_guard<std::mutex> lock(c.mu);
+// The function `name` of an embedded code object on `device`, its module loaded once; c.mu held.
+static int code_function(CodeCache& c, int device, const void* code, size_t code_size,
+                         const char* name, tg_function* fn, bool* loaded) {
   CodeKey key{code, code_size, device};
   auto it = c.modules.find(key);
   hipModule_t m;
   if (it == c.modules.end()) {
     TG_HIP(hipModuleLoadData(&m, code), "hipModuleLoadData");
     c.modules.emplace(key, m);
+    if (loaded) *loaded = true;
   } else {
     m = it->second;
   }
@@ -271,6 +268,25 @@ int tg_code_function(const void* code, size_t code_size, const char* name,
   c.functions.emplace(fkey, f);
   *fn = f;
   return 0;
+}
+
+int tg_code_function(const void* code, size_t code_size, const char* name,
+                     tg_function* fn) {
+  return tg_code_function_beside(code, code_size, nullptr, 0, name, fn);
+}
+
+int tg_code_function_beside(const void* code, size_t code_size, const void* other,
+                            size_t other_size, const char* name, tg_function* fn) {
+  if (!code || !code_size || !name || !fn) return fail(-1, "tg_code_function: null argument");
+  int device = 0;
+  TG_HIP(hipGetDevice(&device), "hipGetDevice");
+  CodeCache& c = code_cache();
+  std::lock_guard<std::mutex> lock(c.mu);
+  bool loaded = false;
+  const int rc = code_function(c, device, code, code_size, name, fn, &loaded);
+  if (rc != 0 || !loaded || !other) return rc;
+  tg_function beside;
+  return code_function(c, device, other, other_size, name, &beside, nullptr);
 }
 
 int tg_code_release(const void* code, size_t code_size) {

@@ -51,6 +51,8 @@ class Variant:
         self.launch.argtypes = _SIGNATURES[kernel_name]
         self.launch.restype = None
         self.lib.tgv_function.restype = ctypes.c_void_p
+        self.lib.tgv_function_for.restype = ctypes.c_void_p
+        self.lib.tgv_function_for.argtypes = [ctypes.c_int64]
         self.lib.tgv_geometry.argtypes = [ctypes.c_int64] * 4 + [
             ctypes.POINTER(ctypes.c_int64), ctypes.POINTER(ctypes.c_int32),
             ctypes.POINTER(ctypes.c_int32)]
@@ -58,9 +60,11 @@ class Variant:
         self._async = None
 
     # -- launch geometry / raw function (for timing harnesses) ------------ #
-    def function(self) -> int:
+    def function(self, K: Optional[int] = None) -> int:
+        """The variant's kernel, right at any K; with ``K`` the one that a launch with K dense
+        columns (16-byte aligned operands) takes."""
         _rt.lib().tg_clear_error()
-        fn = self.lib.tgv_function()
+        fn = self.lib.tgv_function() if K is None else self.lib.tgv_function_for(K)
         if not fn:
             _rt.check_status("tgv_function")
             raise _rt.TileGenHipError("tgv_function returned null")

@@ -118,6 +118,18 @@ def _atomic_compile(cmd_head: List[str], src: str, out: str, tail: List[str]) ->
             os.unlink(tmp)
 
 
+def _code_object(gen: "_codegen.GeneratedKernel", path: str, opts: List[str]) -> Tuple[bytes, str]:
+    if os.path.exists(path):
+        with open(path, "rb") as fh:
+            return fh.read(), "code object from cache"
+    code, log = _rt.rtc_compile(gen.source, gen.filename, opts)
+    tmp = path + ".tmp%d" % os.getpid()
+    with open(tmp, "wb") as fh:
+        fh.write(code)
+    os.replace(tmp, path)
+    return code, log
+
+
 def _compile_hip(gen: "_codegen.GeneratedKernel", workdir: str) -> Tuple[str, str]:
     opts = hiprtc_options()
     key = hashlib.sha1("\0".join([gen.source, gen.host_source] + opts).encode()).hexdigest()[:20]
@@ -125,20 +137,19 @@ def _compile_hip(gen: "_codegen.GeneratedKernel", workdir: str) -> Tuple[str, st
     cdir = cache_dir()
     so_path = os.path.join(cdir, stem + ".so")
     co_path = os.path.join(cdir, stem + ".co")
-    if os.path.exists(so_path) and os.path.exists(co_path):
+    small = "{SMALL_OBJECT}" in gen.host_source
+    small_path = os.path.join(cdir, stem + "_small.co")
+    if os.path.exists(so_path) and os.path.exists(co_path) and (
+            not small or os.path.exists(small_path)):
         return so_path, "cached %s (hipRTC %s)" % (so_path, hip_arch())
-    if os.path.exists(co_path):
-        with open(co_path, "rb") as fh:
-            code = fh.read()
-        rtc_log = "code object from cache"
-    else:
-        code, rtc_log = _rt.rtc_compile(gen.source, gen.filename, opts)
-        tmp = co_path + ".tmp%d" % os.getpid()
-        with open(tmp, "wb") as fh:
-            fh.write(code)
-        os.replace(tmp, co_path)
+    code, rtc_log = _code_object(gen, co_path, opts)
     host = gen.host_source.replace("{CODE_SIZE}", str(len(code))).replace(
         "{CODE_OBJECT}", _bytes_as_c(code))
+    if small:
+        code2, log2 = _code_object(gen, small_path, opts + ["-DTG_SMALL"])
+        host = host.replace("{SMALL_SIZE}", str(len(code2))).replace(
+            "{SMALL_OBJECT}", _bytes_as_c(code2))
+        rtc_log += log2
     os.makedirs(workdir, exist_ok=True)
     # per-process file name: concurrent builds of one variant never read a
     # launcher source another process is still writing
