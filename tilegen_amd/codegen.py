@@ -3128,6 +3128,7 @@ def _spmm_wave_calls(w: _W, low: Lowering, geo: LaunchGeometry, out_name: str, b
     w("if (threadIdx.x < 2) s_col[threadIdx.x] = cc;")
     w("__syncthreads();")
     TPR, SLOTS = max(1, low.threads_per_row), B // max(1, low.threads_per_row)
+    W2 = 2 * TPR * V     # columns of tg_spmm_rows' two slices
     # The rule's lines, each side measured (us a launch; 16 nonzeros per row over 100 k rows
     # unless said otherwise, 16-row tiles on one wave; skewed matrices on 128-row tiles):
     #   B rows of whole 128-byte lines: lane groups 98 / 217 at K = 64 / 128, one wave per
@@ -3136,24 +3137,37 @@ def _spmm_wave_calls(w: _W, low: Lowering, geo: LaunchGeometry, out_name: str, b
     #     comes from the Infinity Cache at 6.9 TB/s, its rate for streams.
     #   other K: a 16-column slice straddles two lines, which the next slice fetches again:
     #     lane groups 190 / 340 / 534 at K = 33 / 63 / 130, one wave per nonzero (each line
-    #     once) 86 / 146 / 271, 7.2 TB/s at K = 130.  Up to 32 columns a wave would be half
-    #     empty: both slices of a nonzero at once, 114 -> 77 at K = 30, 73 -> 54 at K = 20.
+    #     once) 86 / 146 / 266, 7.2 TB/s at K = 130.  Up to 32 columns a wave would be half
+    #     empty: both slices of a nonzero at once, 114 -> 77 at K = 30, 73 -> 55 at K = 20.
+    #   one pass of a lane group covers K: neither has anything to add, as nothing is fetched
+    #     twice: 64-lane groups, unroll 4, two slices 203 and one 74 at K = 20, one wave per
+    #     nonzero 87 and one slice 84 at K = 33.
     #   columns close together (a band): B comes from L2 and the lane groups wait for their
     #     index loads: one wave per nonzero 80 against 96 at K = 64, 137 against 196 at 128
     #     (7 diagonals, 200 k rows).
-    #   skewed tiles: runs of equal length per wave and helpers for the dwarfing rows 114
-    #     against 353 (power law, K = 64), 92 against 315 (1% of rows 2000 long).
-    #   few waves: 2000 rows 9.7 against 15.4 at K = 64 and 9.9 against 18.2 at K = 33;
-    #     10000 rows (625 waves) 20.9 against 30.4.
+    #   skewed tiles: runs of equal length per wave and helpers for the dwarfing rows 102
+    #     against 322 (power law, K = 64), 79 against 324 (1% of rows 2000 long).
     w("const bool lines = ((%s & 15) == 0) && ((((unsigned long long)%s) & 127) == 0);"
       % (kext, b_name))
-    w("// a grid of under 8 waves per CU waits for latency: two column slices and 3 nonzeros of")
-    w("// a row at a time")
-    w("const bool few = tn * %d < %d && %s <= 64;" % (WAVES, 8 * 256, kext))
-    w("bool wave = s_skew || (!lines && %s > 32 && !few);" % kext)
+    w("const bool one = %s <= %d%s;" % (kext, TPR, " * (vec_ok ? 2 : 1)" if V == 2 else ""))
     w("const tg_i64 span = tg_uniform(s_col[1] - s_col[0]);")
-    w("const bool near = %s > 32 && !few && span < 256 && span > -256 && s_ptr[1] > s_ptr[0] + 1;"
-      % kext)
+    w("// a grid of under 8 waves per CU waits for latency: two column slices and 3 nonzeros of")
+    w("// a row at a time, 2000 rows 9.7 us against 15.4 at K = 64 and 9.9 against 18.2 at K = 33")
+    w("const bool small = tn * %d < %d;" % (WAVES, 8 * 256))
+    w("bool near = %s > 32 && !one && !(small && %s <= 64) && span < 256 && span > -256 && "
+      "s_ptr[1] > s_ptr[0] + 1;" % (kext, kext))
+    if WAVES <= 2 and W2 >= 32:
+        w("// (over 64 columns too where the alternative is the lane groups' or a band's: 8000 rows,")
+        w("// K = 256, 71 against 107; 7 diagonals, 8000 rows, K = 128, 12.3 against 18.9.  One wave")
+        w("// per nonzero stays ahead: 24000 rows, K = 130, 60 against 69)")
+        w("const bool few = small && !one && (%s <= 64 || lines || near);" % kext)
+    else:
+        w("// (a slice that is half empty costs more than it saves where a workgroup's waves share")
+        w("// a CU: tiles of 128 rows on 512 lanes, 24000 rows, K = 48 43 against 37)")
+        w("const bool few = small && !one && %s <= 64 && (!lines || %s %% %d == 0);"
+          % (kext, kext, W2))
+    w("bool wave = s_skew || (!lines && !one && %s > 32 && !few);" % kext)
+    w("near = near && !few;")
     w("wave = wave || near;")
     w.open("if (wave)")
     w("if (t_rows <= 0) return;")
@@ -3172,11 +3186,11 @@ def _spmm_wave_calls(w: _W, low: Lowering, geo: LaunchGeometry, out_name: str, b
     w("else %s" % call(2, 2, 4))
     w("return;")
     w.close()
-    w.open("if (!lines || few)")
+    w.open("if (!one && (!lines || few))")
     w("#pragma unroll 1")
     w("for (tg_i64 kb = 0; kb < %s; kb += %d) tg_spmm_rows<%d, %d, 2, %d, %d>(indices, data, %s, "
       "%s, %s, row0, (int)t_rows, s_ptr, kb);"
-      % (kext, 2 * TPR * V, TPR, V, 3, SLOTS, b_name, out_name, kext))
+      % (kext, W2, TPR, V, 3, SLOTS, b_name, out_name, kext))
     w("return;")
     w.close()
 
