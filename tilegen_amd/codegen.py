@@ -3439,10 +3439,13 @@ def _hip_sparse_out(w: _W, plan: Plan, low: Lowering, bound: str, geo: LaunchGeo
     # over 64 columns (the runs' one nonzero per wave) a dense block's rows lose the V rows
     # that neighbours share: 261 us by runs, 196 a row per wave side by side (4x4 blocks, 4 per
     # row, K = 130); up to 64 the runs are ahead there too (63 against 119 at K = 33)
-    if V == 1:
-        forms = [(16, 16, 1, 1), (32, 32, 1, 1), (64, 64, 1, 1), (128, 64, 1, 2), (0, 64, 1, 4)]
-    else:
-        forms = [(16, 16, 1, 1), (32, 16, 2, 1), (64, 32, 2, 1), (128, 64, 2, 1), (0, 64, 2, 2)]
+    # (K up to, lanes per nonzero, columns per load, loads per lane).  32 lanes of several loads
+    # past 64 columns: two nonzeros' V rows per instruction, and no lanes without a column where
+    # K just passes 64 or 128.  Against 64 lanes of one load (K <= 128) or two: uniform, 24 k
+    # rows, K = 66 / 128 / 130 / 256 32.0 / 54.5 / 60.2 / 114 us against 38.1 / 56.5 / 64.7 / 121,
+    # power law, 100 k rows, K = 66 / 130 87 / 152 against 91 / 156.
+    forms = [(16, 16, 1, 1), (32, 16, 2, 1), (64, 32, 2, 1), (128, 32, 2, 2), (192, 32, 2, 3),
+             (0, 32, 2, 4)]
     w("// equal runs of the launch's nonzeros per wave, whatever rows they lie in")
     w("const tg_i64 tg_gw = (tg_i64)blockIdx.x * %d + wave, tg_nw = (tg_i64)gridDim.x * %d;"
       % (WAVES, WAVES))
@@ -3633,10 +3636,10 @@ __device__ __forceinline__ bool tg_blocked(const tg_i64* __restrict__ indptr,
 // are in flight, and their dot products are summed over the lanes together (tg_sums).  Rows
 // and columns of 64 positions are kept one per lane.  Nonzeros of one row share the row's U
 // slice; where the batch spans rows each loads its own, which L1 holds.
-// Bound by the V gathers: 1.6 M nonzeros over 130 columns (uniform, 100 k rows) take 293 us,
-// 1.84 GB in lines from the Infinity Cache at 6.3 TB/s; a power law's 0.8 M take 163 where a
-// wave per row took 730 (its rows of 5000 on one workgroup), 55 against 444 at K = 33.  2 to 8
-// nonzeros' loads at once keep the kernel under 128 VGPRs, the chunked path's 4 waves per SIMD.
+// Bound by the V gathers: 1.6 M nonzeros over 130 columns (uniform, 100 k rows) take 262 us,
+// 1.84 GB in lines from the Infinity Cache at 7.0 TB/s; a power law's 0.8 M take 151 where a
+// wave per row took 640 (its rows of 5000 on one workgroup), 56 against 444 at K = 33.  1 to 8
+// nonzeros' loads at once keep the kernel at 128 VGPRs, 4 waves per SIMD.
 template <int G, int CL, int E, class F>
 __device__ __forceinline__ void tg_sddmm_run(
     const tg_i64* __restrict__ indptr, const tg_i64* __restrict__ indices,
@@ -3706,10 +3709,12 @@ __device__ __forceinline__ void tg_sddmm_run(
             #pragma unroll
             for (int c = 0; c < CL; ++c) t += tg_cols<CL>::get(x, c) * tg_cols<CL>::get(y, c);
           } else {
-            const int k = e * G * CL + q * CL;
+            const int k = q * CL;
+            int past = left - e * G * CL;
+            if (E > 2) asm volatile("" : "+s"(past));   // masks made anew: kept, they spill
             #pragma unroll
             for (int c = 0; c < CL; ++c)
-              t = (c == CL - 1 ? k < left : k + CL <= left)
+              t = (c == CL - 1 ? k < past : k + CL <= past)
                   ? t + tg_cols<CL>::get(x, c) * tg_cols<CL>::get(y, c) : t;
           }
         };
@@ -3719,7 +3724,7 @@ __device__ __forceinline__ void tg_sddmm_run(
           cols ur[E];
           #pragma unroll
           for (int e = 0; e < E; ++e) ur[e] = *(const cols*)(Uk + rf * K * 8 + ko[e]);
-          constexpr int H = E == 1 ? 8 : 4;   // at once: 8 of the widest form pass 128 VGPRs
+          constexpr int H = E == 1 ? 8 : E == 4 ? 2 : 4;   // at once
           #pragma unroll
           for (int h = 0; h < 8; h += H) {
             cols v[H][E];
@@ -3736,9 +3741,10 @@ __device__ __forceinline__ void tg_sddmm_run(
               #pragma unroll
               for (int e = 0; e < E; ++e)
                 if (e * G * CL < left) fma(acc[h + u], e, ur[e], v[u][e]);
+            if (E > 2) __builtin_amdgcn_sched_barrier(0);   // else past 128 VGPRs
           }
         } else {
-          constexpr int H = E == 1 ? 4 : 2;
+          constexpr int H = E == 1 ? 4 : E == 4 ? 1 : 2;
           #pragma unroll
           for (int h = 0; h < 8; h += H) {
             cols x[H][E], v[H][E];
