@@ -3080,9 +3080,25 @@ def _spmm_helpers(w: _W, plan: Plan, low: Lowering, geo: LaunchGeometry, out_nam
     w("// the band path's do, each XCD takes a contiguous eighth of the tiles, so that a band's")
     w("// neighbouring tiles share its L2: 7 diagonals, 200 k rows, K = 45 52.8 -> 42.6 us, K = 64")
     w("// 49.2 -> 44.4.  100 k rows of 16 uniform columns, K = 64, take 101 us so and 98 in turn.")
+    w("// Only where the edges of the eighths lie within 1/128 of the nonzeros of equal shares:")
+    w("// rows ordered by length would leave most of the work to one XCD (36 in the first eighth of")
+    w("// 100 k rows, 4 in the others, K = 64 176 us so and 102 in turn)")
     w("const unsigned tb = blockIdx.x - n_help, xq = tn / 8, xr = tn % 8, xc = tb % 8;")
-    w("const tg_i64 row0 = (tg_i64)(nnz <= 8 * %s ? xc * xq + (xc < xr ? xc : xr) + tb / 8 : tb) * %d;"
-      % (plan.row_extent, TR))
+    w("const tg_i64 rlast = row_end > 0 ? row_end : 0;")
+    w("const bool low = nnz <= 8 * %s;" % plan.row_extent)
+    w("tg_i64 row0 = (tg_i64)(low ? xc * xq + (xc < xr ? xc : xr) + tb / 8 : tb) * %d;" % TR)
+    w("tg_i64 pv = indptr[row0 + threadIdx.x < rlast ? row0 + threadIdx.x : rlast];")
+    w.open("if (low)")
+    w("const unsigned l = threadIdx.x < 8 ? threadIdx.x : 8;   // lane l: the pointer ahead of eighth l")
+    w("const tg_i64 edge = (tg_i64)(l * xq + (l < xr ? l : xr)) * %d;" % TR)
+    w("const tg_i64 ev = indptr[edge < rlast ? edge : rlast];")
+    w("const tg_i64 e0 = tg_lane_read(ev, 0), all = tg_lane_read(ev, 8) - e0;")
+    w("const tg_i64 off = 8 * (ev - e0) - l * all;")
+    w.open("if (__ballot(16 * (off < 0 ? -off : off) > all))")
+    w("row0 = (tg_i64)tb * %d;" % TR)
+    w("pv = indptr[row0 + threadIdx.x < rlast ? row0 + threadIdx.x : rlast];")
+    w.close()
+    w.close()
 
 
 def _spmm_wave_calls(w: _W, low: Lowering, geo: LaunchGeometry, out_name: str, b_name: str,
@@ -3103,8 +3119,9 @@ def _spmm_wave_calls(w: _W, low: Lowering, geo: LaunchGeometry, out_name: str, b
         w("__shared__ double s_band[%d];" % (16 * SPMM_BAND))
     w("const tg_i64 t_rows = row_end - row0 < %d ? row_end - row0 : %d;" % (TR, TR))
     w("if (threadIdx.x == 0) { s_nh = 0; s_skew = 0; }")
-    w("const tg_i64 rlast = row_end > 0 ? row_end : 0;")
-    w("tg_i64 pv = indptr[row0 + threadIdx.x < rlast ? row0 + threadIdx.x : rlast];")
+    if not spmm_band(geo):
+        w("const tg_i64 rlast = row_end > 0 ? row_end : 0;")
+        w("tg_i64 pv = indptr[row0 + threadIdx.x < rlast ? row0 + threadIdx.x : rlast];")
     w("// the first and the last column of the tile's first row, in flight over the staging")
     w("tg_i64 cc = 0;")
     w.open("if (threadIdx.x < 64)")
