@@ -3633,18 +3633,23 @@ __device__ __forceinline__ tg_i64 tg_row_of(const tg_i64* __restrict__ indptr, c
   return lo;
 }
 
-// Whether neighbouring rows mostly name the same columns (dense blocks): 16 pairs of rows
-// across the matrix, the same ones for every wave, at least 6 of which begin alike.
+// Whether neighbouring rows mostly name the same columns (dense blocks): 8 pairs of rows
+// across the matrix, the same ones for every wave, at least 3 of which have more than one
+// nonzero and the same first and middle column.  By the first column alone a hub passes for
+// blocks: a power law with column 0 in every row, 100 k rows, K = 65 / 130 605 / 644 us so,
+// 81 / 135 now.  16 pairs cost blocks of 24 k rows 1.3% more, K = 65.
 __device__ __forceinline__ bool tg_blocked(const tg_i64* __restrict__ indptr,
                                            const tg_i64* __restrict__ indices, const tg_i64 R) {
   const int i = threadIdx.x & 63;
-  tg_i64 r = R * i / 16 + (i & 3);
-  const bool in = i < 16 && r + 2 <= R;
+  tg_i64 r = R * i / 8 + (i & 3);
+  const bool in = i < 8 && r + 2 <= R;
   if (!in) r = 0;
   const tg_i64 p0 = indptr[r], p1 = indptr[r + 1], p2 = indptr[in ? r + 2 : r + 1];
-  bool same = in && p1 > p0 && p2 > p1;
-  if (same) same = indices[p0] == indices[p1];
-  return __builtin_amdgcn_readfirstlane(__builtin_popcountll(__ballot(same))) >= 6;
+  bool same = in && p1 - p0 > 1 && p2 - p1 > 1;
+  if (same)
+    same = indices[p0] == indices[p1] &&
+           indices[p0 + (p1 - p0) / 2] == indices[p1 + (p2 - p1) / 2];
+  return __builtin_amdgcn_readfirstlane(__builtin_popcountll(__ballot(same))) >= 3;
 }
 
 // SDDMM by runs: wave gw of nw takes the positions [a, b), an equal share of the launch's
