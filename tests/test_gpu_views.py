@@ -183,6 +183,16 @@ def test_spmm_and_sddmm_row_block(parity, hip_ready):
     _check_block("sddmm", TUNED["c5"], parity, K=16)
 
 
+@pytest.mark.parametrize("K", [33, 64, 130])
+@pytest.mark.parametrize("cfg", [TUNED["c4"], TUNED["c5"], TEST_SCHEDULES[0], TEST_SCHEDULES[3]],
+                         ids=["c4", "c5", "single lanes", "8 waves"])
+def test_spmm_and_sddmm_row_block_of_many_columns(cfg, K, hip_ready):
+    """The same past 16 columns and the chunked SDDMM path: helpers, runs of nonzeros and the
+    choice of paths take their positions from the row pointers, whatever nnz says."""
+    _check_block("spmm", cfg, 1, K=K)
+    _check_block("sddmm", cfg, 1, K=K)
+
+
 @pytest.mark.parametrize("cfg", SCRATCH_FORMS, ids=[schedule_id(c) for c in SCRATCH_FORMS])
 def test_undercounted_nnz_then_a_correct_launch(cfg, hip_ready):
     """A launch told a third of the nonzeros (or one) gives the full product, and
