@@ -102,8 +102,8 @@ def illegal_reason(cfg: Config) -> Optional[str]:
 
 def sddmm_group_per_row(cfg: Config, K: int) -> bool:
     """Whether the SDDMM variant takes its chunked path at this K (one lane
-    group per row, K covered by one group's registers) rather than one wave
-    per row."""
+    group per row, K covered by one group's registers) rather than equal runs
+    of nonzeros per wave, or one wave per row of dense blocks."""
     tpr, V = cfg.threads_per_row, 2 if cfg.vector_width >= 2 else 1
     return K <= tpr * V * max(1, cfg.unroll) and (V == 1 or K % 2 == 0)
 
@@ -121,8 +121,10 @@ def illegal_reason_for(kernel: str, cfg: Config, K: int = 8) -> Optional[str]:
             per, what = cfg.block_size // cfg.threads_per_row, "lane group"
         else:
             per, what = cfg.block_size // _WAVE, "wave"
+        # past the chunked path the tile sets the rows of a dense block's workgroup and, for
+        # the runs of nonzeros, how many waves share them
         if cfg.tile_size < per or cfg.tile_size > 8 * per:
-            return ("sddmm runs one row per %s at K=%d: tile_size must be 1..8 x %d"
+            return ("sddmm tiles hold 1..8 rows per %s at K=%d: tile_size must be 1..8 x %d"
                     % (what, K, per))
         return None
     r = illegal_reason(cfg)

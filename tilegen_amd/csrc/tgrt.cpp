@@ -370,8 +370,8 @@ int tg_launch_ordered(const void* order_key, tg_function fn, int64_t grid, int32
     return tg_launch(fn, grid, block, lds_bytes, args, n_args, stream, 0);
   }
   OrderTable& t = order_table();
-  // held across wait, launch and record, so two host threads cannot both
-  // launch after the same recorded end
+  // held across the wait and the launch that carries the event, so that two host
+  // threads cannot both launch after the same launch's end
   std::lock_guard<std::mutex> lock(t.mu);
   OrderState& st = t.keys[std::make_pair(order_key, device)];
   if (!st.done) TG_HIP(hipEventCreateWithFlags(&st.done, hipEventDisableTiming), "hipEventCreate");
