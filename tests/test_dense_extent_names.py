@@ -37,6 +37,25 @@ def test_launcher_passes_the_kernels_dense_extent(make, F):
     assert re.search(r"tgv_geometry\(M, N, %s, nnz, &grid" % F, host)
 
 
+@pytest.mark.parametrize("make", [_spmm, _sddmm], ids=["spmm", "sddmm"])
+def test_grid_is_tgv_geometrys_and_needs_k(make, tmp_path):
+    from tilegen_amd.verify import compile_generated
+    for cfg in (WIDE, TUNED["c4"], TUNED["c5"], Config()):
+        gen = generate(make("K"), cfg, "hip", outdir=str(tmp_path))
+        lib = ctypes.CDLL(compile_generated(gen, "hip", str(tmp_path))[0])
+        lib.tgv_geometry.argtypes = [ctypes.c_int64] * 4 + [ctypes.c_void_p] * 3
+        g, b, l = ctypes.c_int64(), ctypes.c_int32(), ctypes.c_int32()
+        for M in (0, 1, 63, 700, 100003, 1 << 31):
+            for nnz in (0, 1, 5000, 16 * M):
+                for K in (0, 1, 16, 17, 32, 33, 64, 65):
+                    lib.tgv_geometry(M, 9, K, nnz, ctypes.byref(g), ctypes.byref(b),
+                                     ctypes.byref(l))
+                    assert gen.geometry.grid(M, nnz, K) == g.value, (cfg.short(), M, nnz, K)
+        if cfg.tile_size > 1:
+            with pytest.raises(ValueError, match="depends on K"):
+                gen.geometry.grid(700, 5000)
+
+
 def _operands(A, F, out):
     rng = np.random.default_rng(4)
     M, N = A.shape

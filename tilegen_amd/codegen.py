@@ -222,7 +222,10 @@ class LaunchGeometry:
     helper_div: int = 0
     helper_K: int = 0
 
-    def grid(self, rows: int, nnz: int = 0, K: int = 64) -> int:
+    def grid(self, rows: int, nnz: int = 0, K: Optional[int] = None) -> int:
+        """Workgroups of a launch; tiled SpMM and SDDMM need K, which decides their helpers."""
+        if K is None and (self.helper_div or self.helper_K):
+            raise ValueError("the grid of a tiled SpMM or SDDMM variant depends on K")
         if rows <= 0:
             return 0
         if self.stream:
@@ -3914,9 +3917,11 @@ def _hip_sparse_out_fast(w: _W, plan: Plan, TPR: int, U: int, V: int, SLOTS: int
         w.open("if (row0 < 0)")
         w("// Helper e: when the row that holds position e ch dwarfs its tile, that row's positions")
         w("// from there to the next boundary, and those before it when this is the row's first.")
-        w("// On a power law (100 k rows, 800 k nonzeros) 512 of them take K = 64 from 147 to 95 us")
-        w("// (256: 119, 128: 145) and K = 8 from 120 to 68; rows of like length cost them one")
-        w("// probe of the row pointers, 0.3 us of 26 at K = 8")
+        w("// On a power law (100 k rows, 800 k nonzeros) 512 of them take K = 64 from 141 to 105 us")
+        w("// (256: 113, 128: 144) and K = 14 from 116 to 78.  Where rows are alike they probe the row")
+        w("// pointers and leave: up to 2000 tiles nothing that a run resolves, 16 uniform nonzeros")
+        w("// per row, 20 k rows, K = 14 / 64 7.4 -> 7.8 / 18.1 -> 18.5, 60 k rows 23.0 -> 23.5 / 68.8")
+        w("// -> 69.5")
         w("const tg_i64 tg_ch = 1LL << tg_chs, tg_P = (tg_i64)blockIdx.x << tg_chs;")
         w("if (row_end <= 0) return;")
         w("const tg_i64 tg_pb = tg_uniform(indptr[0]), tg_pe = tg_uniform(indptr[row_end]);")
@@ -4107,8 +4112,8 @@ def emit_hip_host(kernel: Kernel, config: Config) -> str:
 
     ``{CODE_OBJECT}`` and ``{CODE_SIZE}`` are replaced by the compiled bytes
     when the variant is built (``{SMALL_OBJECT}`` and ``{SMALL_SIZE}`` by those compiled with
-    TG_SMALL, where ``small_kernel_test`` gives the launches that take them).  The launcher exports the reference ABI
-    (synchronous, device pointers, errors reported through ``tg_last_error``)
+    TG_SMALL, where ``small_kernel_test`` gives the launches that take them).  The launcher
+    exports the reference ABI (synchronous, device pointers, errors reported through ``tg_last_error``)
     plus ``tgv_geometry``, ``tgv_function`` and ``tgv_launch_async`` for
     harnesses that time the kernel on their own stream.  Variants that combine
     row pieces through module scratch (``module_scratch``) launch through
@@ -4176,7 +4181,7 @@ void* tgv_function_for(int64_t K) { (void)K; return tgv_function(); }
 
 static const unsigned char tg_code[{CODE_SIZE}] = {{CODE_OBJECT}};%(small_code)s
 
-/* the runtime caches the loaded module by tg_code's address: drop that entry
+/* the runtime caches a loaded module by its code's address: drop that entry
    when this library is unloaded, before another can be mapped there */
 __attribute__((destructor)) static void tgv_unload(void) {
   tg_code_release(tg_code, sizeof(tg_code));%(release)s

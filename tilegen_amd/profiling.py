@@ -107,7 +107,7 @@ def case_plan(steps: int, warmup: int, case_iters: int
         M, N, nnz = A.shape[0], A.shape[1], int(A.nnz)
         k = run_pipeline(standard_kernels()[bc.kernel], TUNED[case], backend="hip")
         geo = launch_geometry(_plan(k), _lowering(k))
-        grid = geo.grid(M, nnz) * geo.block
+        grid = geo.grid(M, nnz, bc.K) * geo.block
         if case == HEADLINE:
             timed = steps
             n = 1 + warmup + steps + warmup + steps
