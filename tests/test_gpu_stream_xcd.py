@@ -14,7 +14,7 @@ from tests.test_gpu_parity import _check
 from tests.util import csr
 from tilegen_amd.codegen import STREAM_XCD, generate
 from tilegen_amd.dsl import standard_kernels
-from tilegen_amd.schedules import STREAM_TEST_SCHEDULES
+from tilegen_amd.schedules import STREAM_TEST_SCHEDULES, TUNED
 
 CFG = STREAM_TEST_SCHEDULES[1]      # ranges of 64: the most workgroups per nonzero
 CH = CFG.block_size * CFG.unroll
@@ -31,6 +31,25 @@ def test_every_range_has_one_workgroup():
         b = np.arange(G)
         e = b % 8 * (G // 8) + np.minimum(b % 8, G % 8) + b // 8
         assert np.array_equal(np.sort(e), b), G
+
+
+def test_the_upper_line_counts_nonzeros():
+    for cfg in STREAM_TEST_SCHEDULES + [TUNED["c3a"], TUNED["c3b"]]:
+        ch = cfg.block_size * cfg.unroll
+        src = generate(standard_kernels()["spmv"], cfg, "hip", write=False).source
+        assert "gridDim.x > %du ?" % ((1 << 22) // ch) in src, cfg.short()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", ["c3a", "c3b"])
+def test_wider_ranges_at_the_upper_line(case, hip_ready):
+    ch = TUNED[case].block_size * TUNED[case].unroll
+    for G in ((1 << 22) // ch, (1 << 22) // ch + 1, (1 << 22) // ch + 7):
+        nnz, rng = (G - 1) * ch + 5, np.random.default_rng(G)
+        ip = np.r_[0, np.sort(rng.integers(0, nnz + 1, nnz // 8)), nnz].astype(np.int64)
+        A = csr(ip.size - 1, 700, ip, rng.integers(0, 700, nnz), rng.uniform(-1, 1, nnz))
+        print("[gpu] spmv %s stream grid %d" % (case, G), flush=True)
+        _check("spmv", TUNED[case], A, K=1, label="%s grid %d" % (case, G))
 
 
 @pytest.mark.gpu

@@ -906,8 +906,8 @@ def spmm_part(block: int, V: int) -> int:
 # staged in LDS, 8 bytes each)
 STREAM_MAX_CHUNK = 8192
 # Stream ranges are dealt to the XCDs in contiguous eighths up to this many (two per CU)
-# and past this many (two rounds of seven per CU)
-STREAM_XCD = (512, 3584)
+# and past this many of 64 nonzeros, the smallest, or as many nonzeros of a wider range
+STREAM_XCD = (512, 65536)
 
 
 def stream_chunk(low: Lowering) -> int:
@@ -1622,15 +1622,17 @@ __device__ tg_i64 tg_st_row(const tg_i64* __restrict__ indptr, tg_i64 R, tg_i64 
         w("// sub-buffer may be only 8-byte aligned, which takes the per-element loads")
         w("const bool pair_ok = ((((unsigned long long)indices) | "
           "((unsigned long long)data)) & 15) == 0;")
-    w("// Workgroups go to the 8 XCDs in turn.  With few ranges or many, each XCD takes a")
+    w("// Workgroups go to the 8 XCDs in turn.  With few ranges or many nonzeros, each XCD takes a")
     w("// contiguous eighth of them, so that neighbouring ranges' row pointers and search")
-    w("// probes share one L2: 1 M power-law rows, 7760 ranges of 1024, 121.0 -> 108.5 us;")
-    w("// 400 k rows of 16, 6250 ranges, 49.4 -> 48.3; 20000 rows of 4 with 1% of 2000, 235")
-    w("// ranges of 2048, 6.6 -> 6.1.  Between the lines range e stays with workgroup e:")
-    w("// 776 ranges took 11.4 us dealt this way against 10.7, 1563 ranges 15.6 against 14.6,")
-    w("// 3106 ranges 36.1 against 35.8.")
+    w("// probes share one L2: 20000 rows of 4 with 1% of 2000, 235 ranges of 2048, 6.6 -> 6.1 us;")
+    w("// 400 k rows of 16, 6250 ranges of 1024, 49.4 -> 48.3.  What gains at the top is a matrix")
+    w("// that no L2 holds, whatever its ranges: power law, 768 k rows (6.1 M nonzeros) in ranges")
+    w("// of 1024 / 2048 / 4096 83.2 -> 74.9 / 77.9 -> 72.5 / 85.3 -> 81.8, 512 k rows 45.0 -> 44.8")
+    w("// (2048), 384 k rows 34.5 -> 35.0 (1024), 37.6 -> 39.5 (512).  Between the lines range e")
+    w("// stays with workgroup e: 256 k rows, 2000 ranges of 1024, 24.5 us dealt this way and 23.3")
     w("const unsigned xq = gridDim.x / 8, xr = gridDim.x % 8, xc = blockIdx.x % 8;")
-    w("const tg_i64 e = gridDim.x <= %du || gridDim.x > %du ?" % STREAM_XCD)
+    w("const tg_i64 e = gridDim.x <= %du || gridDim.x > %du ?"
+      % (STREAM_XCD[0], STREAM_XCD[1] * 64 // CH))
     w("    xc * xq + (xc < xr ? xc : xr) + blockIdx.x / 8 : blockIdx.x;")
 
     def phase1(positions: bool) -> None:
