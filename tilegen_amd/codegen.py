@@ -7,8 +7,9 @@ translation unit per variant; every variant exposes the reference ABI
 backend "hip"
     ``GeneratedKernel.source`` is device code only (one ``extern "C"
     __global__`` kernel plus small wave64 helpers), compiled at run time by
-    hipRTC for gfx950.  ``GeneratedKernel.host_source`` is a C launcher that
-    embeds the compiled code object and exports ``launch_<name>`` with the
+    hipRTC for gfx950 (spmm and sddmm a second time with TG_SMALL, for the path
+    of few columns alone).  ``GeneratedKernel.host_source`` is a C launcher that
+    embeds the compiled code objects and exports ``launch_<name>`` with the
     reference argument list, plus ``tgv_geometry``/``tgv_function`` for timing
     harnesses.  The device code is written for CDNA4, not translated:
 
