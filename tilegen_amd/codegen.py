@@ -224,9 +224,8 @@ class LaunchGeometry:
     helper_K: int = 0
 
     def grid(self, rows: int, nnz: int = 0, K: Optional[int] = None) -> int:
-        """Workgroups of a launch; tiled SpMM and SDDMM need K, which decides their helpers."""
-        if K is None and (self.helper_div or self.helper_K):
-            raise ValueError("the grid of a tiled SpMM or SDDMM variant depends on K")
+        """Workgroups of a launch.  Tiled SpMM and SDDMM add helpers by K; without it, the tiles
+        alone, a grid that is right at any K."""
         if rows <= 0:
             return 0
         if self.stream:
@@ -234,6 +233,8 @@ class LaunchGeometry:
         g = (int(rows) + self.rows_per_block - 1) // self.rows_per_block
         if self.nnz_chunk:
             g += max(0, int(nnz)) // self.nnz_chunk + 1
+        if K is None:
+            return g
         if self.helper_div and K > SPMM_WAVE_K:
             hr = spmm_helper_rows(int(rows), self.helper_div)
             help_ = SPMM_SLICES * ((int(rows) + hr - 1) // hr)
