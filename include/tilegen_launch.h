@@ -82,8 +82,8 @@ void* tgv_function(void);                  /* the variant's kernel, current devi
  * tgv_function's is right at any K */
 void* tgv_function_for(int64_t K);
 const char* tgv_kernel_name(void);         /* "spmv", "spmm", ... */
-/* grid and block of a launch; *lds_bytes is the dynamic LDS to pass, always 0:
- * every generated kernel declares its LDS statically */
+/* grid and block of a launch (K 0: of tgv_function's kernel at any K); *lds_bytes is the
+ * dynamic LDS to pass, always 0: every generated kernel declares its LDS statically */
 int tgv_geometry(int64_t M, int64_t N, int64_t K, int64_t nnz, int64_t* grid,
                  int32_t* block, int32_t* lds_bytes);
 

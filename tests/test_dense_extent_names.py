@@ -1,6 +1,6 @@
 """SpMM and SDDMM whose dense extent is not called "K": the launcher asks for the grid of the
-extent the kernel compares, and a launch with a grid of the tiles alone (no helper workgroups)
-still writes every tile."""
+extent the kernel compares, and a launch on the grid that is given for no K in particular writes
+every tile."""
 
 from __future__ import annotations
 
@@ -38,7 +38,7 @@ def test_launcher_passes_the_kernels_dense_extent(make, F):
 
 
 @pytest.mark.parametrize("make", [_spmm, _sddmm], ids=["spmm", "sddmm"])
-def test_grid_is_tgv_geometrys_or_the_tiles_alone(make, tmp_path):
+def test_grid_is_tgv_geometrys(make, tmp_path):
     from tilegen_amd.verify import compile_generated
     for cfg in (WIDE, TUNED["c4"], TUNED["c5"], Config()):
         gen = generate(make("K"), cfg, "hip", outdir=str(tmp_path))
@@ -51,7 +51,7 @@ def test_grid_is_tgv_geometrys_or_the_tiles_alone(make, tmp_path):
                     lib.tgv_geometry(M, 9, K, nnz, ctypes.byref(g), ctypes.byref(b),
                                      ctypes.byref(l))
                     assert gen.geometry.grid(M, nnz, K) == g.value, (cfg.short(), M, nnz, K)
-        assert gen.geometry.grid(700, 5000) == -(-700 // gen.geometry.rows_per_block)
+        assert gen.geometry.grid(700, 5000) == gen.geometry.grid(700, 5000, 0)
 
 
 def _operands(A, F, out):
@@ -62,8 +62,8 @@ def _operands(A, F, out):
 
 
 def _run(name, cfg, A, F, outdir, raw_grid=None):
-    """The launch_<name> of a library whose extent is "F" or its kernel on another grid: with
-    ``raw_grid`` K tgv_geometry's for that K, with "tiles" the tiles alone."""
+    """The launch_<name> of a library whose extent is "F" or its kernel on tgv_geometry's
+    grid for ``raw_grid`` columns."""
     from tilegen_amd import runtime as rt
     from tilegen_amd.verify import compile_generated
     gen = generate((_spmm if name == "spmm" else _sddmm)("F"), cfg, "hip", outdir=str(outdir))
@@ -83,10 +83,8 @@ def _run(name, cfg, A, F, outdir, raw_grid=None):
         else:
             g, b, l = ctypes.c_int64(), ctypes.c_int32(), ctypes.c_int32()
             lib.tgv_geometry.argtypes = [ctypes.c_int64] * 4 + [ctypes.c_void_p] * 3
-            lib.tgv_geometry(A.shape[0], A.shape[1], 0, 0, ctypes.byref(g),
+            lib.tgv_geometry(A.shape[0], A.shape[1], raw_grid, 0, ctypes.byref(g),
                              ctypes.byref(b), ctypes.byref(l))
-            if raw_grid == "tiles":
-                g.value = gen.geometry.grid(A.shape[0], A.nnz)
             lib.tgv_function.restype = ctypes.c_void_p
             rt.time_launches(lib.tgv_function(), g.value, b.value, l.value, [vals], 0, 1)
         return bufs[-1].to_host(), dense
@@ -96,7 +94,7 @@ def _run(name, cfg, A, F, outdir, raw_grid=None):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("raw_grid", [None, 0, "tiles"])
+@pytest.mark.parametrize("raw_grid", [None, 0])
 @pytest.mark.parametrize("cfg", [TUNED["c4"], WIDE, TUNED["c5"]], ids=["c4", "wide", "c5"])
 def test_every_tile_is_written(cfg, raw_grid, tmp_path, hip_ready):
     A = ragged(61, 900, 700, 12, empty_every=7, long_rows=[(0, 690), (400, 650), (899, 600)])

@@ -224,8 +224,9 @@ class LaunchGeometry:
     helper_K: int = 0
 
     def grid(self, rows: int, nnz: int = 0, K: Optional[int] = None) -> int:
-        """Workgroups of a launch.  Tiled SpMM and SDDMM add helpers by K; without it, the tiles
-        alone, a grid that is right at any K."""
+        """Workgroups of a launch.  Tiled SpMM and SDDMM add helpers by K; without it, or at 0, a
+        grid that is right at any K."""
+        K = K or 0
         if rows <= 0:
             return 0
         if self.stream:
@@ -233,9 +234,7 @@ class LaunchGeometry:
         g = (int(rows) + self.rows_per_block - 1) // self.rows_per_block
         if self.nnz_chunk:
             g += max(0, int(nnz)) // self.nnz_chunk + 1
-        if K is None:
-            return g
-        if self.helper_div and K > SPMM_WAVE_K:
+        if self.helper_div and (K > SPMM_WAVE_K or K <= 0):
             hr = spmm_helper_rows(int(rows), self.helper_div)
             help_ = SPMM_SLICES * ((int(rows) + hr - 1) // hr)
             if (g + help_) * self.block <= 0xFFFFFFFF:
@@ -3010,8 +3009,9 @@ def _spmm_helpers(w: _W, plan: Plan, low: Lowering, geo: LaunchGeometry, out_nam
          SPMM_HELP_MAX))
     w("hr = hr < 64 ? 64 : hr;")
     w("unsigned n_help = (unsigned)((%s + hr - 1) / hr) * %d;" % (plan.row_extent, NS))
-    w("// none past one launch's work-items, or where the caller's grid is for the tiles alone")
-    w("if (gridDim.x != tn + n_help) n_help = 0;")
+    w("// none past one launch's work-items.  (gridDim would tell too, but its hidden arguments cost")
+    w("// a launch of 20 to 50 us 0.2 to 0.8)")
+    w("if (((tg_i64)tn + n_help) * %d > 0xFFFFFFFFLL) n_help = 0;" % B)
     w("__shared__ unsigned long long s_hrow[%d];  // a helper's rows, one bit each" % (SPMM_HELP_MAX // 64))
     w.open("if (blockIdx.x < n_help)")
     w("// Helper: of its hr rows, those over %d nonzeros and over 4 times their tile's" % LH)
@@ -3173,7 +3173,8 @@ def _spmm_wave_calls(w: _W, low: Lowering, geo: LaunchGeometry, out_name: str, b
     #     against 322 (power law, K = 64), 79 against 324 (1% of rows 2000 long).
     w("const bool lines = ((%s & 15) == 0) && ((((unsigned long long)%s) & 127) == 0);"
       % (kext, b_name))
-    w("const bool one = %s <= %d%s;" % (kext, TPR, " * (vec_ok ? 2 : 1)" if V == 2 else ""))
+    w("const bool one = %s;" % ("%s <= %d%s" % (kext, TPR, " * (vec_ok ? 2 : 1)" if V == 2 else "")
+                                if TPR * V > SPMM_WAVE_K else "false"))
     w("const tg_i64 span = tg_uniform(s_col[1] - s_col[0]);")
     w("// a grid of under 8 waves per CU waits for latency: two column slices and 3 nonzeros of")
     w("// a row at a time, 2000 rows 9.7 us against 15.4 at K = 64 and 9.9 against 18.2 at K = 33")
@@ -3443,8 +3444,8 @@ def _hip_sparse_out(w: _W, plan: Plan, low: Lowering, bound: str, geo: LaunchGeo
         w("const tg_i64 tg_per = nnz > 0 ? nnz >> tg_hs : 0;")
         w("const int tg_chs = tg_per < %d ? %d : 64 - __builtin_clzll((unsigned long long)tg_per);"
           % (SDDMM_HELP_MIN, SDDMM_HELP_MIN.bit_length() - 1))
-        w("// none past one launch's work-items, or where the caller's grid is for the tiles alone")
-        w("if (gridDim.x != tg_tn + tg_n_help) tg_n_help = 0;")
+        w("if ((tg_tn + tg_n_help) * %d > 0xFFFFFFFFLL) tg_n_help = 0;  // past one launch's work-items"
+          % B)
         w("const tg_i64 row0 = ((tg_i64)blockIdx.x - tg_n_help) * %d;" % TR)
     else:
         w("const tg_i64 row0 = (tg_i64)blockIdx.x * %d;" % TR)
@@ -4248,7 +4249,7 @@ int tgv_launch_async(void* stream, %(params)s) {
                   "\n  if (*grid > 0) *grid += (nnz > 0 ? nnz : 0) / %d + 1;"
                   % geo.nnz_chunk) if geo.nnz_chunk and not geo.stream else
                  ("\n  /* helper workgroups ahead of the tiles, for rows that dwarf their tile */"
-                  "\n  if (*grid > 0 && K > %d) {"
+                  "\n  if (*grid > 0 && (K > %d || K <= 0)) {"
                   "\n    int64_t hr = (rows / %d + 63) / 64 * 64;"
                   "\n    hr = hr < 64 ? 64 : hr > %d ? %d : hr;"
                   "\n    const int64_t help = %d * ((rows + hr - 1) / hr);"
