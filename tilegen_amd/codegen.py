@@ -3183,9 +3183,12 @@ def _spmm_wave_calls(w: _W, low: Lowering, geo: LaunchGeometry, out_name: str, b
       "s_ptr[1] > s_ptr[0] + 1;" % (kext, kext))
     if WAVES <= 2 and W2 >= 32:
         w("// (over 64 columns too where the alternative is the lane groups' or a band's: 8000 rows,")
-        w("// K = 256, 71 against 107; 7 diagonals, 8000 rows, K = 128, 12.3 against 18.9.  One wave")
-        w("// per nonzero stays ahead: 24000 rows, K = 130, 60 against 69)")
-        w("const bool few = small && !one && (%s <= 64 || lines || near);" % kext)
+        w("// K = 256, 71 against 107; 7 diagonals, 8000 rows, K = 128, 12.3 against 18.9.  Other K up")
+        w("// to 192 while tiles and columns are few, 2500 rows, K = 70 / 150 13.8 / 21.6 against one")
+        w("// wave per nonzero's 23.5 / 31.6, 8000 rows 25.8 / 45.4 against 29.7 / 45.2; it takes 256")
+        w("// columns at once: 2500 rows, K = 250, 50 against 40)")
+        w("const bool few = small && !one && (%s <= 64 || lines || near || (%s <= 192 && tn * %d * %s "
+          "< 65536));" % (kext, kext, WAVES, kext))
     else:
         w("// (a slice that is half empty costs more than it saves where a workgroup's waves share")
         w("// a CU: tiles of 128 rows on 512 lanes, 24000 rows, K = 48 43 against 37)")
