@@ -3737,14 +3737,24 @@ __device__ __forceinline__ void tg_sddmm_run(
           ko[e] = (unsigned)((k + CL <= left ? k : left - CL) + (int)(kb - kbase)) * 8u;
         }
         // a slice of columns: whole (every lane's count), partly past K or all past K
+        // (of three slices and more each is summed by itself first: fewer roundings of the growing
+        // sum, for an error like that of twice the lanes with chains half as long; four have no
+        // registers left for it in a slice that ends inside)
         auto fma = [&](double& t, int e, const cols& x, const cols& y) {
-          if ((e + 1) * G * CL <= left) {
+          const bool whole = (e + 1) * G * CL <= left;
+          const int k = q * CL;
+          int past = left - e * G * CL;
+          if (E > 2) asm volatile("" : "+s"(past));   // masks made anew: kept, they spill
+          if (whole) {
+            double p = E > 2 ? 0.0 : t;
             #pragma unroll
-            for (int c = 0; c < CL; ++c) t += tg_cols<CL>::get(x, c) * tg_cols<CL>::get(y, c);
+            for (int c = 0; c < CL; ++c) p += tg_cols<CL>::get(x, c) * tg_cols<CL>::get(y, c);
+            t = E > 2 ? t + p : p;
+          } else if (E == 3) {
+            double p = tg_cols<CL>::get(x, CL - 1) * tg_cols<CL>::get(y, CL - 1);
+            p = k + CL <= past ? p + tg_cols<CL>::get(x, 0) * tg_cols<CL>::get(y, 0) : p;
+            t = k < past ? t + p : t;
           } else {
-            const int k = q * CL;
-            int past = left - e * G * CL;
-            if (E > 2) asm volatile("" : "+s"(past));   // masks made anew: kept, they spill
             #pragma unroll
             for (int c = 0; c < CL; ++c)
               t = (c == CL - 1 ? k < past : k + CL <= past)
