@@ -3935,11 +3935,10 @@ def _hip_sparse_out_fast(w: _W, plan: Plan, TPR: int, U: int, V: int, SLOTS: int
         w.open("if (row0 < 0)")
         w("// Helper e: when the row that holds position e ch dwarfs its tile, that row's positions")
         w("// from there to the next boundary, and those before it when this is the row's first.")
-        w("// On a power law (100 k rows, 800 k nonzeros) 512 of them take K = 64 from 141 to 105 us")
-        w("// (256: 113, 128: 144) and K = 14 from 116 to 78.  Where rows are alike they probe the row")
-        w("// pointers and leave: up to 2000 tiles nothing that a run resolves, 16 uniform nonzeros")
-        w("// per row, 20 k rows, K = 14 / 64 7.4 -> 7.8 / 18.1 -> 18.5, 60 k rows 23.0 -> 23.5 / 68.8")
-        w("// -> 69.5")
+        w("// On a power law (100 k rows, 800 k nonzeros) 512 of them take K = 64 from 142 to 106 us")
+        w("// (256: 113, 128: 147) and K = 14 from 116 to 79.  Where rows are alike they probe the row")
+        w("// pointers and leave: 16 uniform nonzeros per row, 20 k rows, K = 14 / 64 7.3 -> 7.6 / 17.1")
+        w("// -> 17.2, 60 k rows 23.5 -> 23.6 / 68.5 -> 69.3")
         w("const tg_i64 tg_ch = 1LL << tg_chs, tg_P = (tg_i64)blockIdx.x << tg_chs;")
         w("if (row_end <= 0) return;")
         w("const tg_i64 tg_pb = tg_uniform(indptr[0]), tg_pe = tg_uniform(indptr[row_end]);")
